@@ -10,6 +10,7 @@
 //   total, pad; pairs/all_pairs.cuh:29-114 all-pairs path; common/traversal.cuh:12-147 visit
 //   order and periodic images; runtime/entry_points.cu:127-508 launch order and gating.
 
+#include <algorithm>
 #include <climits>
 #include <limits>
 #include <mutex>
@@ -119,10 +120,13 @@ template <typename T>
 __global__ void __launch_bounds__(kBlock) assign_bins_kernel(
     const T* __restrict__ positions, const index_t* __restrict__ dims,
     const T* __restrict__ widths, index_t num_atoms, index_t* __restrict__ atom_bin,
-    index_t* __restrict__ bin_counts, const index_t* rebuild, const index_t* status)
+    index_t* __restrict__ bin_counts, index_t* __restrict__ full_slices, const index_t* rebuild,
+    const index_t* status)
 {
     const std::int64_t atom = static_cast<std::int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
     if (atom >= num_atoms || !rebuilding(rebuild, status)) return;
+    // the full rows' slice widths start at 0: the count raises each to its widest row
+    if (full_slices != nullptr && atom % kWave == 0) full_slices[atom / kWave] = 0;
     const T* p = positions + 3 * atom;
     const index_t nx = dims[0], ny = dims[1];
     const index_t bin = axis_bin(p[0], widths[0], nx) +
@@ -197,7 +201,7 @@ __global__ void __launch_bounds__(kBlock) order_bins_kernel(
     }
 }
 
-// ---- pair visit -----------------------------------------------------------------------------
+// ---- pair visit: a lane per center, for sparse grids ----------------------------------------
 
 // Visits, for sorted center `center`, every candidate in the reference's order (neighbor bins
 // z, y, x from -1 to +1; candidates ascending) and calls visit(neighbor, after) for each one
@@ -369,6 +373,453 @@ __global__ void __launch_bounds__(kBlock) fill_pairs_kernel(
     visit_grid<T, kFull>(sp, bin_offsets, atom_bin[sorted_ids[center]], dims[0], dims[1], dims[2],
                          cell[0], cell[1], cell[2], radius_squared, static_cast<index_t>(center),
                          visit);
+}
+
+// ---- pair search ----------------------------------------------------------------------------
+
+// Centers a wave tests against each chunk of 64 candidates: with 8 in fp32 the scalar registers
+// no longer hold the centers and their masks (2.24 ms a rebuild at 2,097,152 atoms, radius 1.1
+// nm, against 2.17).
+constexpr int kSearchCenters = 4;
+constexpr int kSearchRanges = 32;  // lanes that may hold a range of candidates (18 are used)
+
+// How a candidate's vector is formed, uniform over a wave's centers (one bin).
+constexpr int kSearchPlain = 0;    // every candidate bin inside the box: center - candidate
+constexpr int kSearchShifted = 1;  // some bins across a face: the near-face coordinate shifted
+constexpr int kSearchImage = 2;    // an axis of fewer than three bins: minimum image per pair
+
+template <typename T>
+struct SearchArgs
+{
+    const T* sp;                  // [N, 3] positions in slot order
+    const index_t* sorted_ids;    // slot -> atom
+    const index_t* bin_offsets;
+    const index_t* dims;
+    const T* cell;
+    T radius_squared;
+    std::int64_t bin_slots;
+    // count
+    index_t* pair_counts;
+    index_t* full_counts;
+    index_t* full_slices;         // zero before the count; the fill reads their prefix sums
+    // fill
+    const index_t* pair_offsets;
+    index_t* pairs;
+    std::int64_t capacity;
+    index_t* full_index;
+    std::int64_t full_capacity;
+    const index_t* rebuild;
+    const index_t* status;
+};
+
+// The candidate ranges of a bin, one per lane, in the reference's visit order (bins z, y, x from
+// -1 to +1): consecutive bins along x are consecutive slots, so a (z, y) row is one range, or two
+// where it crosses an x face. `shift` holds two bits per axis: 1 below the box (the candidate
+// moves down by L), 2 above it (the center does).
+struct SearchRange
+{
+    index_t lo, length;
+    int shift;
+};
+
+template <typename T>
+__device__ __forceinline__ SearchRange search_range(const SearchArgs<T>& a, index_t hx, index_t hy,
+                                                    index_t hz, index_t nx, index_t ny, index_t nz,
+                                                    int lane)
+{
+    SearchRange r{0, 0, 0};
+    const int span_y = ny >= 3 ? 3 : ny, span_z = nz >= 3 ? 3 : nz;
+    const int row = lane / 2, part = lane % 2;
+    if (row >= span_y * span_z) return r;
+    const int oy = row % span_y, oz = row / span_y;
+    const index_t ry = ny >= 3 ? hy + oy - 1 : oy, rz = nz >= 3 ? hz + oz - 1 : oz;
+    const index_t by = ry < 0 ? ry + ny : (ry >= ny ? ry - ny : ry);
+    const index_t bz = rz < 0 ? rz + nz : (rz >= nz ? rz - nz : rz);
+    r.shift = (ry < 0 ? 4 : (ry >= ny ? 8 : 0)) | (rz < 0 ? 16 : (rz >= nz ? 32 : 0));
+    index_t first = 0, last = -1;
+    if (nx < 3)
+    {
+        if (part == 0) last = nx - 1;
+    }
+    else if (hx == 0)
+    {
+        first = part == 0 ? nx - 1 : 0;
+        last = part == 0 ? nx - 1 : 1;
+        if (part == 0) r.shift |= 1;
+    }
+    else if (hx == nx - 1)
+    {
+        first = part == 0 ? nx - 2 : 0;
+        last = part == 0 ? nx - 1 : 0;
+        if (part == 1) r.shift |= 2;
+    }
+    else if (part == 0)
+    {
+        first = hx - 1;
+        last = hx + 1;
+    }
+    if (last < first) return r;
+    const index_t base = nx * (by + ny * bz);
+    r.lo = a.bin_offsets[base + first];
+    r.length = a.bin_offsets[base + last + 1] - r.lo;
+    return r;
+}
+
+// A tile of a bin's candidates in LDS, in visit order, without those too far from the bin's atoms
+// to pair with any of them.
+constexpr int kSearchWaves = 4;
+constexpr int kSearchPerLane = 4;
+
+template <typename T>
+struct SearchTile
+{
+    static constexpr int kRaw = kSearchWaves * kWave * kSearchPerLane;  // candidates read per tile
+    T x[kRaw], y[kRaw], z[kRaw];
+    index_t slot[kRaw], id[kRaw], shift[kRaw];
+    index_t start[kSearchRanges], to_slot[kSearchRanges], range_shift[kSearchRanges];
+    index_t kept[kSearchWaves * kSearchPerLane];
+    T box[6];
+};
+
+// Candidates [base, base + kRaw) of the bin's ranges into the tile; returns how many it holds.
+// `reach` bounds the distance from the box of the bin's atoms at which a candidate can still be
+// a neighbor (image mode keeps every one).
+template <typename T, bool kFill, int kMode>
+__device__ __forceinline__ index_t stage_candidates(const SearchArgs<T>& a,
+                                                    SearchTile<T>& tile, index_t base,
+                                                    index_t total, T lx, T ly, T lz, T reach_squared)
+{
+    using Tile = SearchTile<T>;
+    constexpr int kThreads = kSearchWaves * kWave;
+    const int lane = lane_id();
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    T px[kSearchPerLane], py[kSearchPerLane], pz[kSearchPerLane];
+    index_t slot[kSearchPerLane], id[kSearchPerLane], shift[kSearchPerLane];
+    std::uint64_t keep[kSearchPerLane];
+    // every read of the tile before any use: a turn waits for memory once
+#pragma unroll
+    for (int u = 0; u < kSearchPerLane; ++u)
+    {
+        const index_t t = base + u * kThreads + static_cast<index_t>(threadIdx.x);
+        int r = 0;
+#pragma unroll
+        for (int step = kSearchRanges / 2; step > 0; step >>= 1)
+            if (tile.start[r + step] <= t) r += step;
+        slot[u] = t < total ? tile.to_slot[r] + t : -1;
+        shift[u] = kMode == kSearchShifted ? tile.range_shift[r] : 0;
+    }
+#pragma unroll
+    for (int u = 0; u < kSearchPerLane; ++u)
+    {
+        const index_t from = slot[u] < 0 ? 0 : slot[u];
+        px[u] = a.sp[3LL * from];
+        py[u] = a.sp[3LL * from + 1];
+        pz[u] = a.sp[3LL * from + 2];
+        id[u] = kFill ? a.sorted_ids[from] : 0;
+    }
+#pragma unroll
+    for (int u = 0; u < kSearchPerLane; ++u)
+    {
+        bool take = slot[u] >= 0;
+        if (kMode != kSearchImage)
+        {
+            T qx = px[u], qy = py[u], qz = pz[u];
+            if (kMode == kSearchShifted)
+            {
+                const int code = shift[u];
+                px[u] = px[u] + ((code & 1) != 0 ? -lx : T(0));
+                py[u] = py[u] + ((code & 4) != 0 ? -ly : T(0));
+                pz[u] = pz[u] + ((code & 16) != 0 ? -lz : T(0));
+                qx = px[u] + ((code & 2) != 0 ? lx : T(0));
+                qy = py[u] + ((code & 8) != 0 ? ly : T(0));
+                qz = pz[u] + ((code & 32) != 0 ? lz : T(0));
+            }
+            const T gx = fmax(fmax(tile.box[0] - qx, qx - tile.box[3]), T(0));
+            const T gy = fmax(fmax(tile.box[1] - qy, qy - tile.box[4]), T(0));
+            const T gz = fmax(fmax(tile.box[2] - qz, qz - tile.box[5]), T(0));
+            take = take && squared(gx, gy, gz) < reach_squared;
+        }
+        keep[u] = ballot(take);
+        if (lane == 0) tile.kept[u * kSearchWaves + wave] = __popcll(keep[u]);
+    }
+    __syncthreads();
+    index_t count = 0;
+    index_t before[kSearchPerLane];
+#pragma unroll
+    for (int u = 0; u < kSearchPerLane; ++u)
+#pragma unroll
+        for (int w = 0; w < kSearchWaves; ++w)
+        {
+            if (w == wave) before[u] = count;
+            count += tile.kept[u * kSearchWaves + w];
+        }
+#pragma unroll
+    for (int u = 0; u < kSearchPerLane; ++u)
+        if ((keep[u] >> lane) & 1ull)
+        {
+            const int at = before[u] + bits_below(keep[u]);
+            tile.x[at] = px[u];
+            tile.y[at] = py[u];
+            tile.z[at] = pz[u];
+            tile.slot[at] = slot[u];
+            if (kFill) tile.id[at] = id[u];
+            if (kMode == kSearchShifted) tile.shift[at] = shift[u];
+        }
+    __syncthreads();
+    static_assert(Tile::kRaw == kThreads * kSearchPerLane, "one candidate per lane and turn");
+    return __builtin_amdgcn_readfirstlane(count);
+}
+
+// The centers of one wave: kSearchCenters consecutive slots, their coordinates and running
+// places scalar.
+template <typename T>
+struct SearchGroup
+{
+    T x[kSearchCenters], y[kSearchCenters], z[kSearchCenters];
+    index_t id[kSearchCenters];
+    index_t half[kSearchCenters];  // count: pairs so far; fill: the next column
+    index_t row[kSearchCenters];   // count: neighbors so far; fill: the next full entry
+};
+
+// The group against the tile's candidates, 64 a turn. A turn's hits of a center are a ballot: its
+// bits count them, and rank each hit in the center's columns (half list: candidates after the
+// center) and in its full row, so a turn's hits go out as one run from a scalar address.
+template <typename T, bool kFull, bool kFill, int kMode>
+__device__ __forceinline__ void search_tile(const SearchArgs<T>& a,
+                                            const SearchTile<T>& tile, index_t count,
+                                            index_t first, int live, T lx, T ly, T lz,
+                                            SearchGroup<T>& c)
+{
+    const int lane = lane_id();
+    for (index_t chunk = 0; chunk < count; chunk += kWave)
+    {
+        const index_t at = chunk + lane < count ? chunk + lane : count - 1;
+        const T px = tile.x[at], py = tile.y[at], pz = tile.z[at];
+        const index_t slot = tile.slot[at];
+        const index_t id = kFill ? tile.id[at] : 0;
+        const int shift = kMode == kSearchShifted ? tile.shift[at] : 0;
+        const std::uint64_t valid =
+            count - chunk >= kWave ? ~0ull : (1ull << (count - chunk)) - 1ull;
+        // candidates after every center, and those that are centers of this group themselves
+        const std::uint64_t beyond = valid & ballot(slot >= first + live);
+        const std::uint64_t own = valid & ballot(slot >= first && slot < first + live);
+#pragma unroll
+        for (int g = 0; g < kSearchCenters; ++g)
+        {
+            if (g >= live) break;
+            T dx, dy, dz;
+            if (kMode == kSearchImage)
+            {
+                dx = minimum_image(c.x[g], px, lx);
+                dy = minimum_image(c.y[g], py, ly);
+                dz = minimum_image(c.z[g], pz, lz);
+            }
+            else if (kMode == kSearchShifted)
+            {
+                dx = ((shift & 2) != 0 ? c.x[g] - lx : c.x[g]) - px;
+                dy = ((shift & 8) != 0 ? c.y[g] - ly : c.y[g]) - py;
+                dz = ((shift & 32) != 0 ? c.z[g] - lz : c.z[g]) - pz;
+            }
+            else
+            {
+                dx = c.x[g] - px;
+                dy = c.y[g] - py;
+                dz = c.z[g] - pz;
+            }
+            std::uint64_t hits = valid & ballot(squared(dx, dy, dz) < a.radius_squared);
+            std::uint64_t after = hits & beyond;
+            if (own != 0)
+            {
+                hits &= ~ballot(slot == first + g);
+                after = hits & ballot(slot > first + g);
+            }
+            if (kFill)
+            {
+                // an overflowing build (which the status reports) writes up to the capacity
+                if (after != 0)
+                {
+                    const std::uint32_t rank = bits_below(after);
+                    const std::int64_t room = a.capacity - c.half[g];
+                    if (((after >> lane) & 1ull) && static_cast<std::int64_t>(rank) < room &&
+                        c.half[g] >= 0)
+                    {
+                        index_t* column = a.pairs + c.half[g];
+                        column[rank] = c.id[g];
+                        column[a.capacity + rank] = id;
+                    }
+                    c.half[g] += __popcll(after);
+                }
+                if (kFull && hits != 0)
+                {
+                    const std::uint32_t step = bits_below(hits) * kWave;
+                    const std::int64_t room = a.full_capacity - c.row[g];
+                    if (((hits >> lane) & 1ull) && static_cast<std::int64_t>(step) < room &&
+                        c.row[g] >= 0)
+                    {
+                        index_t* entry = a.full_index + c.row[g];
+                        entry[step] = id;
+                    }
+                    c.row[g] += __popcll(hits) * kWave;
+                }
+            }
+            else
+            {
+                c.half[g] += __popcll(after);
+                if (kFull) c.row[g] += __popcll(hits);
+            }
+        }
+    }
+}
+
+template <typename T, bool kFull, bool kFill, int kMode>
+__device__ __forceinline__ void search_bin(const SearchArgs<T>& a, SearchTile<T>& tile,
+                                           index_t begin, index_t end, index_t total)
+{
+    constexpr int kCenters = kSearchCenters;
+    using Tile = SearchTile<T>;
+    const int lane = lane_id();
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const T lx = a.cell[0], ly = a.cell[1], lz = a.cell[2];
+    // a candidate this far from the box of the bin's atoms pairs with none of them, whatever the
+    // rounding of its image
+    const T radius = sqrt(a.radius_squared);
+    const T longest = fmax(lx, fmax(ly, lz));
+    const T reach = radius * T(1.001) + T(16) * std::numeric_limits<T>::epsilon() * longest;
+    const T reach_squared = reach * reach;
+    index_t staged = -1, count = 0;
+    for (index_t round = begin; round < end; round += kSearchWaves * kCenters)
+    {
+        const index_t first = round + wave * kCenters;
+        const int live = first >= end ? 0 : (end - first < kCenters ? end - first : kCenters);
+        const index_t mine = first + (lane < live ? lane : 0);
+        SearchGroup<T> c;
+        if (live > 0)
+        {
+            const T mx = a.sp[3LL * mine], my = a.sp[3LL * mine + 1], mz = a.sp[3LL * mine + 2];
+            const index_t id = kFill ? a.sorted_ids[mine] : 0;
+            const index_t column = kFill ? a.pair_offsets[mine] : 0;
+            const index_t entry =
+                kFill && kFull ? a.full_slices[mine / kWave] + mine % kWave : 0;
+#pragma unroll
+            for (int g = 0; g < kCenters; ++g)
+            {
+                c.x[g] = read_lane(mx, g);
+                c.y[g] = read_lane(my, g);
+                c.z[g] = read_lane(mz, g);
+                c.id[g] = read_lane(id, g);
+                c.half[g] = read_lane(column, g);
+                c.row[g] = read_lane(entry, g);
+            }
+        }
+        for (index_t base = 0; base < total; base += Tile::kRaw)
+        {
+            if (staged != base)
+            {
+                if (staged >= 0) __syncthreads();
+                count = stage_candidates<T, kFill, kMode>(a, tile, base, total, lx, ly, lz,
+                                                                  reach_squared);
+                staged = base;
+            }
+            if (live > 0)
+                search_tile<T, kFull, kFill, kMode>(a, tile, count, first, live, lx, ly,
+                                                            lz, c);
+        }
+        if (!kFill)
+        {
+            index_t half = 0, full = 0;
+#pragma unroll
+            for (int g = 0; g < kCenters; ++g)
+            {
+                half = lane == g ? c.half[g] : half;
+                full = lane == g ? c.row[g] : full;
+            }
+            if (lane < live)
+            {
+                a.pair_counts[mine] = half;
+                if (kFull)
+                {
+                    a.full_counts[mine] = full;
+                    atomicMax(a.full_slices + mine / kWave, full * kWave);
+                }
+            }
+        }
+    }
+}
+
+// A block per bin. The candidates of a bin are the same for all its atoms: the block reads them
+// once into LDS, leaving out those out of reach of the box of the bin's atoms (a quarter of the
+// 27 bins' atoms at 28 atoms a bin), and each wave tests its centers against them. Bound by the
+// issue of vector and scalar instructions (about 11 of each per center and 64 candidates). A
+// lane per center, each writing columns of its own, wrote the lists 4 bytes to a line. A rebuild
+// at 2,097,152 atoms, radius 1.1 nm, full list: 6.9 -> 2.2 ms (the fill 5.8 -> 1.36, the count
+// 1.05 -> 0.72); a fill of 4,096 atoms, whose 64 waves left the chip idle, 140 -> 13 us.
+template <typename T, bool kFull, bool kFill>
+__global__ void __launch_bounds__(kSearchWaves * kWave) search_pairs_kernel(SearchArgs<T> a)
+{
+    __shared__ SearchTile<T> tile;
+    if (!rebuilding(a.rebuild, a.status)) return;
+    const std::int64_t bin = blockIdx.x;
+    const index_t nx = a.dims[0], ny = a.dims[1], nz = a.dims[2];
+    if (bin >= static_cast<std::int64_t>(nx) * ny * nz || bin >= a.bin_slots - 1) return;
+    const index_t begin = __builtin_amdgcn_readfirstlane(a.bin_offsets[bin]);
+    const index_t end = __builtin_amdgcn_readfirstlane(a.bin_offsets[bin + 1]);
+    if (begin == end) return;
+    const index_t home = static_cast<index_t>(bin);
+    const index_t hx = home % nx, hy = (home / nx) % ny, hz = home / (nx * ny);
+    const int lane = lane_id();
+    // every wave finds the ranges for itself; the first writes them for the staging
+    SearchRange range = search_range(a, hx, hy, hz, nx, ny, nz, lane);
+    if (!kFull && range.lo <= begin)
+    {
+        // a half list alone needs no candidate up to the bin's first atom
+        const index_t cut =
+            range.lo + range.length <= begin + 1 ? range.length : begin + 1 - range.lo;
+        range.lo += cut;
+        range.length -= cut;
+    }
+    const index_t inclusive = wave_inclusive_sum(range.length);
+    const index_t total = read_lane(inclusive, kWave - 1);
+    if (threadIdx.x < kSearchRanges)
+    {
+        tile.start[lane] = inclusive - range.length;
+        tile.to_slot[lane] = range.lo - (inclusive - range.length);
+        tile.range_shift[lane] = range.shift;
+    }
+    // the box of the bin's atoms, found by the first wave
+    if (threadIdx.x < kWave)
+    {
+        T low[3], high[3];
+        for (int axis = 0; axis < 3; ++axis)
+        {
+            low[axis] = std::numeric_limits<T>::max();
+            high[axis] = -std::numeric_limits<T>::max();
+        }
+        for (index_t k = begin + lane; k < end; k += kWave)
+            for (int axis = 0; axis < 3; ++axis)
+            {
+                const T v = a.sp[3LL * k + axis];
+                low[axis] = fmin(low[axis], v);
+                high[axis] = fmax(high[axis], v);
+            }
+        for (int axis = 0; axis < 3; ++axis)
+        {
+            const T l = -wave_max(-low[axis]), h = wave_max(high[axis]);
+            if (lane == 0)
+            {
+                tile.box[axis] = l;
+                tile.box[3 + axis] = h;
+            }
+        }
+    }
+    __syncthreads();
+    const bool image = nx < 3 || ny < 3 || nz < 3;
+    const bool inside = hx > 0 && hx < nx - 1 && hy > 0 && hy < ny - 1 && hz > 0 && hz < nz - 1;
+    if (image)
+        search_bin<T, kFull, kFill, kSearchImage>(a, tile, begin, end, total);
+    else if (inside)
+        search_bin<T, kFull, kFill, kSearchPlain>(a, tile, begin, end, total);
+    else
+        search_bin<T, kFull, kFill, kSearchShifted>(a, tile, begin, end, total);
 }
 
 // ---- all-pairs path -------------------------------------------------------------------------
@@ -568,8 +1019,8 @@ int launch_grid(const T* positions, const ndn_neighbor_buffers& b, const index_t
 {
     const index_t n = static_cast<index_t>(b.num_atoms);
     assign_bins_kernel<T><<<blocks_for(n), kBlock, 0, stream>>>(
-        positions, b.dims, static_cast<const T*>(b.widths), n, b.atom_bin, b.bin_counts, rebuild,
-        b.status);
+        positions, b.dims, static_cast<const T*>(b.widths), n, b.atom_bin, b.bin_counts,
+        b.full_index != nullptr ? b.full_slices : nullptr, rebuild, b.status);
     NDN_LAUNCHED("assign_bins");
     const int scanned = exclusive_scan(b.bin_counts, b.bin_offsets, b.bin_slots, b.scan_temp,
                                        rebuild, b.status, stream);
@@ -583,6 +1034,72 @@ int launch_grid(const T* positions, const ndn_neighbor_buffers& b, const index_t
         static_cast<T*>(b.sorted_positions), rebuild, b.status);
     NDN_LAUNCHED("order_bins");
     return NDN_OK;
+}
+
+// Whether a block per bin searches the grid, or a lane per center. A block stages 27 bins for the
+// centers of one, which pays from about seven atoms a bin (a rebuild of 100,000 atoms, radius
+// 1.0 nm, full list: 283 us against a lane per center's 179 at 4.1 atoms a bin, 229 against 204
+// at 6.4, 213 against 285 at 9.4, 204 against 398 at 14.6); up to 8,192 atoms, whose lanes fill
+// a small part of the chip, from two (3,000 atoms: 85 us against 110 at 2.3).
+bool block_per_bin(std::int64_t atoms, std::int64_t bins)
+{
+    return atoms >= bins * (atoms <= 8192 ? 2 : 7);
+}
+
+// The search over the grid: the count (kFill false) or the fill.
+template <typename T, bool kFill>
+void launch_search(const T* cell, T radius_squared, const ndn_neighbor_buffers& b,
+                   const index_t* rebuild, hipStream_t stream)
+{
+    const std::int64_t bins = b.bin_slots - 1;
+    const index_t n = static_cast<index_t>(b.num_atoms);
+    const T* sp = static_cast<const T*>(b.sorted_positions);
+    const bool full = b.full_index != nullptr;
+    if (!block_per_bin(b.num_atoms, bins))
+    {
+        const unsigned blocks = blocks_for(n);
+        if (kFill && full)
+            fill_pairs_kernel<T, true><<<blocks, kBlock, 0, stream>>>(
+                sp, b.sorted_ids, b.atom_bin, b.bin_offsets, b.dims, cell, b.pair_offsets,
+                radius_squared, n, b.capacity, b.pairs, b.full_slices, b.full_index,
+                b.full_capacity, rebuild, b.status);
+        else if (kFill)
+            fill_pairs_kernel<T, false><<<blocks, kBlock, 0, stream>>>(
+                sp, b.sorted_ids, b.atom_bin, b.bin_offsets, b.dims, cell, b.pair_offsets,
+                radius_squared, n, b.capacity, b.pairs, nullptr, nullptr, 0, rebuild, b.status);
+        else if (full)
+            count_pairs_kernel<T, true><<<blocks, kBlock, 0, stream>>>(
+                sp, b.sorted_ids, b.atom_bin, b.bin_offsets, b.dims, cell, radius_squared, n,
+                b.pair_counts, b.full_counts, b.full_slices, rebuild, b.status);
+        else
+            count_pairs_kernel<T, false><<<blocks, kBlock, 0, stream>>>(
+                sp, b.sorted_ids, b.atom_bin, b.bin_offsets, b.dims, cell, radius_squared, n,
+                b.pair_counts, nullptr, nullptr, rebuild, b.status);
+        return;
+    }
+    SearchArgs<T> a{};
+    a.sp = sp;
+    a.sorted_ids = b.sorted_ids;
+    a.bin_offsets = b.bin_offsets;
+    a.dims = b.dims;
+    a.cell = cell;
+    a.radius_squared = radius_squared;
+    a.bin_slots = b.bin_slots;
+    a.pair_counts = b.pair_counts;
+    a.full_counts = b.full_counts;
+    a.full_slices = b.full_slices;
+    a.pair_offsets = b.pair_offsets;
+    a.pairs = b.pairs;
+    a.capacity = b.capacity;
+    a.full_index = b.full_index;
+    a.full_capacity = b.full_capacity;
+    a.rebuild = rebuild;
+    a.status = b.status;
+    const unsigned blocks = static_cast<unsigned>(bins);
+    if (full)
+        search_pairs_kernel<T, true, kFill><<<blocks, kSearchWaves * kWave, 0, stream>>>(a);
+    else
+        search_pairs_kernel<T, false, kFill><<<blocks, kSearchWaves * kWave, 0, stream>>>(a);
 }
 
 template <typename T>
@@ -620,19 +1137,7 @@ int launch_count(const T* positions, const T* cell, double radius, const ndn_nei
     }
     else
     {
-        const T* sp = static_cast<const T*>(b.sorted_positions);
-        if (full)
-        {
-            count_pairs_kernel<T, true><<<blocks_for(n), kBlock, 0, stream>>>(
-                sp, b.sorted_ids, b.atom_bin, b.bin_offsets, b.dims, cell, r2, n, b.pair_counts,
-                b.full_counts, b.full_slices, rebuild, b.status);
-        }
-        else
-        {
-            count_pairs_kernel<T, false><<<blocks_for(n), kBlock, 0, stream>>>(
-                sp, b.sorted_ids, b.atom_bin, b.bin_offsets, b.dims, cell, r2, n, b.pair_counts,
-                nullptr, nullptr, rebuild, b.status);
-        }
+        launch_search<T, false>(cell, r2, b, rebuild, stream);
         NDN_LAUNCHED("count_pairs");
     }
     int scanned = exclusive_scan(b.pair_counts, b.pair_offsets, b.num_atoms, b.scan_temp, rebuild,
@@ -674,16 +1179,7 @@ int launch_fill(const T* cell, double radius, const ndn_neighbor_buffers& b,
     }
     else
     {
-        const T* sp = static_cast<const T*>(b.sorted_positions);
-        if (full)
-            fill_pairs_kernel<T, true><<<blocks_for(n), kBlock, 0, stream>>>(
-                sp, b.sorted_ids, b.atom_bin, b.bin_offsets, b.dims, cell, b.pair_offsets, r2, n,
-                b.capacity, b.pairs, b.full_slices, b.full_index, b.full_capacity, rebuild,
-                b.status);
-        else
-            fill_pairs_kernel<T, false><<<blocks_for(n), kBlock, 0, stream>>>(
-                sp, b.sorted_ids, b.atom_bin, b.bin_offsets, b.dims, cell, b.pair_offsets, r2, n,
-                b.capacity, b.pairs, nullptr, nullptr, 0, rebuild, b.status);
+        launch_search<T, true>(cell, r2, b, rebuild, stream);
         NDN_LAUNCHED("fill_pairs");
     }
     total_pad_kernel<<<kPadBlocks, kBlock, 0, stream>>>(

@@ -1,0 +1,63 @@
+"""The drop-in list's grid search at its edges: bins with more atoms than the waves of a bin take
+in one turn, empty bins, grids of one, two, three and four bins along an axis, atoms on the faces.
+The pair index [2, C] is compared bit for bit with the oracle's and the full rows with the same
+pairs in both orientations; whole numbers, so no tolerance."""
+
+import numpy as np
+import pytest
+import torch
+
+from nabladyn_amd.neighbors import NeighborList
+from oracle import neighbors as on
+
+pytestmark = pytest.mark.gpu
+
+CELLS = [
+    (4.9, 4.9, 4.9),   # four bins an axis: most bins touch a face
+    (3.7, 6.1, 8.5),   # three bins along x
+    (2.5, 6.1, 3.7),   # two along x: minimum image per pair
+    (8.5, 2.5, 2.5),   # two along y and z
+]
+
+
+def _frame(kind, cell, rng):
+    cell = np.array(cell)
+    if kind == "sparse":  # under two atoms a bin: a lane per center
+        return rng.uniform(0, 1, (40, 3)) * cell
+    if kind == "dense":  # more atoms a bin than 16 waves of 4 or 8 centers take at once
+        return rng.uniform(0, 1, (6000, 3)) * cell
+    if kind == "clustered":  # most atoms in one corner, most bins empty
+        x = rng.normal(0, 0.15, (900, 3))
+        return np.concatenate([x, rng.uniform(0, 1, (60, 3)) * cell])
+    x = rng.uniform(0, 1, (700, 3)) * cell  # "faces": a third of the atoms on a face
+    x[::3, 0] = 0.0
+    x[1::6, 1] = cell[1]
+    return x
+
+
+@pytest.mark.parametrize("dtype,npdt", [(torch.float32, np.float32), (torch.float64, np.float64)])
+@pytest.mark.parametrize("kind", ["sparse", "dense", "clustered", "faces"])
+@pytest.mark.parametrize("cell", CELLS)
+def test_search_at_its_edges(device, dtype, npdt, kind, cell):
+    x = _frame(kind, cell, np.random.default_rng(17))
+    L = np.array(cell).astype(npdt)
+    wrapped, _ = on.wrap(x.astype(npdt), L)
+    ref = on.build(wrapped, L, npdt(1.2), capacity_multiplier=1.25)
+    for full in (True, False):
+        nl = NeighborList(1.0, skin=0.2, full=full)
+        nl.allocate(torch.tensor(x, dtype=dtype, device=device),
+                    torch.tensor(L, dtype=dtype, device=device))
+        assert not nl.all_pairs
+        index = nl.tensors().index.cpu().numpy()
+        np.testing.assert_array_equal(index, ref.pairs)
+        if full:
+            half = on.pair_set(index, nl.num_pairs)
+            rows = nl.tensors().full
+            counts, slices, entries, ids = (v.cpu().numpy() for v in (
+                rows.counts, rows.slices, rows.index, rows.rows))
+            got = np.concatenate([
+                np.stack([np.full(c, ids[r]), entries[slices[r // 64] + r % 64 + 64 * np.arange(c)]],
+                         axis=1) for r, c in enumerate(counts)])
+            both = np.concatenate([half, half[:, ::-1]])
+            key = lambda a: a[np.lexsort((a[:, 1], a[:, 0]))]  # noqa: E731
+            np.testing.assert_array_equal(key(got), key(both))
