@@ -26,6 +26,47 @@ __device__ __forceinline__ double reciprocal<double>(double value)
     return 1.0 / value;
 }
 
+// sqrt(x), correctly rounded: in fp32 the hardware's reciprocal square root with two coupled
+// Newton steps and a last one on the remainder (P. W. Markstein, "Computation of elementary
+// functions on the IBM RISC System/6000 processor", 1990), without the scaling that a library's
+// root does for results near the ends of the range: squared distances are far from them, and one
+// that is not takes the hardware's root.
+template <typename T>
+__device__ __forceinline__ T pair_distance(T x);
+template <>
+__device__ __forceinline__ double pair_distance<double>(double x)
+{
+    return sqrt(x);
+}
+template <>
+__device__ __forceinline__ float pair_distance<float>(float x)
+{
+    const float y = __builtin_amdgcn_rsqf(x);
+    float g = x * y, h = 0.5f * y;
+    const float r = __builtin_fmaf(-h, g, 0.5f);
+    g = __builtin_fmaf(g, r, g);
+    h = __builtin_fmaf(h, r, h);
+    g = __builtin_fmaf(__builtin_fmaf(-g, g, x), h, g);
+    return x > 1e-30f ? g : __builtin_amdgcn_sqrtf(x);
+}
+
+// 1 / x: the hardware reciprocal with one Newton step in fp32, a division in fp64.
+template <typename T>
+__device__ __forceinline__ T refined_reciprocal(T x);
+template <>
+__device__ __forceinline__ double refined_reciprocal<double>(double x)
+{
+    return 1.0 / x;
+}
+template <>
+__device__ __forceinline__ float refined_reciprocal<float>(float x)
+{
+    const float y = __builtin_amdgcn_rcpf(x);
+    const float better = __builtin_fmaf(__builtin_fmaf(-x, y, 1.0f), y, y);
+    // the step makes NaN of the ends of the range (0, infinity), whose reciprocals are exact
+    return better == better ? better : y;
+}
+
 // Row of the unordered type pair (a, b): a(2T - a - 1)/2 + b for a <= b
 // (potential/_lennard_jones/_potential.py:143-151).
 __device__ __forceinline__ int pair_row(std::int64_t a, std::int64_t b, int num_types)

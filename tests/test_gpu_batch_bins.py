@@ -1,0 +1,73 @@
+"""The batched engine's wave per sub-bin at its edges: bins with more atoms than a wave takes
+together (a dense cluster), empty bins, boxes of fewer sub-bins than the stencil along an axis
+(minimum image per pair), atoms on the faces, a single atom; LJ and a table with pairs below its
+first knot. Tolerance as in the batch tests: fp64 1e-12 (tables 3e-12) of the oracle's closed
+forms; fp32 1e-5 of the reference's own fp32 route."""
+
+import numpy as np
+import pytest
+import torch
+
+from nabladyn_amd import batch, potential, workloads
+from oracle import neighbors as on
+from oracle import potentials as op
+from _parity import ROUTE_TOL, lj_route, rel, table_route
+
+pytestmark = pytest.mark.gpu
+
+
+def _frames(rng):
+    lattice = workloads.lattice
+    out = [
+        (lattice((7, 7, 7), (2.5, 2.5, 2.5), 0.02, rng), (2.5, 2.5, 2.5)),  # four half-cutoff bins
+        (lattice((24, 7, 9), (8.5, 2.6, 3.1), 0.02, rng), (8.5, 2.6, 3.1)),
+        (lattice((12, 12, 12), (3.0, 3.0, 3.0), 0.01, rng), (6.0, 6.0, 6.0)),  # one dense octant
+        (lattice((10, 10, 10), (3.7, 3.7, 3.7), 0.02, rng), (3.7, 3.7, 3.7)),
+        (np.full((1, 3), 1.0), (2.5, 2.5, 2.5)),
+    ]
+    faces = out[3][0]
+    faces[::5, 0] = 0.0
+    faces[1::7, 2] = 3.7
+    return out
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("span", [1, 2])
+def test_wave_per_bin_at_its_edges(device, dtype, span):
+    rng = np.random.default_rng(23)
+    table = workloads.lj_table(noise=0.0)[None]
+    systems = []
+    for x, cell in _frames(rng):
+        types = torch.zeros(len(x), dtype=torch.int64, device=device)
+        as_t = lambda v: torch.tensor(np.asarray(v), dtype=dtype, device=device)  # noqa: E731
+        lj = potential.lennard_jones(atom_types=types, sigma=as_t([0.22]), epsilon=as_t([0.996]),
+                                     cutoff=1.0)
+        tab = potential.tabulated(atom_types=types, table=as_t(table), start=as_t([0.3]),
+                                  cutoff=1.2)
+        systems += [(as_t(x), as_t(cell), lj), (as_t(x), as_t(cell), tab)]
+    b = batch.Batch(systems, schedule=("wave", span))
+    energy, forces, virial = b.evaluate()
+    for k, (f, (x, cell, model)) in enumerate(zip(b.split(forces), systems)):
+        cn = cell.cpu().numpy()
+        xw = on.wrap(x.cpu().numpy(), cn)[0]
+        pairs = on.brute_pairs(xw, cn, xw.dtype.type(model.cutoff)).T
+        types = np.zeros(len(xw), np.int64)
+        if isinstance(model, potential.LennardJones):
+            args = (model.sigma.detach().cpu().numpy(), model.epsilon.detach().cpu().numpy())
+            fp64 = op.lj_efw(xw.astype(np.float64), cn.astype(np.float64), pairs, types, *args,
+                             model.cutoff)
+            route = lj_route(xw, cn, pairs, types, *args, model.cutoff)
+        else:
+            args = (model.table.detach().cpu().numpy(), model.start.cpu().numpy())
+            spacing = model.spacing.cpu().numpy()
+            fp64 = op.table_efw(xw.astype(np.float64), cn.astype(np.float64), pairs, types, *args,
+                                model.cutoff, spacing=spacing)
+            route = table_route(xw, cn, pairs, types, *args, spacing, model.cutoff)
+        e0, f0, w0 = fp64 if dtype == torch.float64 else route
+        bar = ROUTE_TOL if dtype == torch.float32 else 3e-12
+        if pairs.shape[1] == 0:
+            assert float(energy[k]) == 0.0 and not f.any() and not virial[k].any()
+            continue
+        assert rel(f.cpu(), f0) <= bar, k
+        assert rel(virial[k].cpu(), w0) <= bar, k
+        assert abs(float(energy[k]) - e0) <= bar * max(1.0, abs(e0)), k
