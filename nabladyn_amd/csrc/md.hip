@@ -523,6 +523,15 @@ __device__ __forceinline__ bool refreshing(const StepArgs<T>& a)
            (a.rebuild[0] != 0 || prune_state(a.header)->refresh != 0);
 }
 
+// Whether a build kernel works on this step: the check asked for a build and no status bit is set
+// but the halo overflow of this very build. Its later phases stay in bounds past that (an atom
+// outside its halo's slots is listed as the sentinel) and report what else overflows.
+template <typename T>
+__device__ __forceinline__ bool building(const StepArgs<T>& a)
+{
+    return a.rebuild[0] != 0 && (a.status[0] & ~kStatusHaloOverflow) == 0;
+}
+
 // The block a kernel body runs as and the number of blocks of its system: the hardware's own in
 // a launch over one system, the system's share in a launch over a batch of systems (the bodies
 // read no blockIdx or gridDim, so a system computes the same bits alone and in a batch).
@@ -928,7 +937,7 @@ template <typename T>
 __device__ __forceinline__ void md_assign_body(const StepArgs<T>& a, const Launch launch,
                                                int forced)
 {
-    if (!forced && !rebuilding(a.rebuild, a.status)) return;
+    if (!forced && !building(a)) return;
     for (std::int64_t slot = static_cast<std::int64_t>(launch.block) * blockDim.x + threadIdx.x;
          slot < a.num_atoms; slot += static_cast<std::int64_t>(launch.blocks) * blockDim.x)
     {
@@ -953,7 +962,7 @@ template <typename T>
 __device__ __forceinline__ void md_scatter_body(const StepArgs<T>& a, const Launch launch,
                                                 int forced)
 {
-    if (!forced && !rebuilding(a.rebuild, a.status)) return;
+    if (!forced && !building(a)) return;
     for (std::int64_t slot = static_cast<std::int64_t>(launch.block) * blockDim.x + threadIdx.x;
          slot < a.num_atoms; slot += static_cast<std::int64_t>(launch.blocks) * blockDim.x)
     {
@@ -989,7 +998,7 @@ template <typename T>
 __device__ __forceinline__ void md_order_body(const StepArgs<T>& a, const Launch launch,
                                               int forced)
 {
-    if (!forced && !rebuilding(a.rebuild, a.status)) return;
+    if (!forced && !building(a)) return;
     for (std::int64_t i = static_cast<std::int64_t>(launch.block) * blockDim.x + threadIdx.x;
          i < a.num_atoms; i += static_cast<std::int64_t>(launch.blocks) * blockDim.x)
     {
@@ -1037,7 +1046,7 @@ template <typename T>
 __device__ __forceinline__ void md_unpack_body(const StepArgs<T>& a, const Launch launch,
                                                int forced)
 {
-    if (!forced && !rebuilding(a.rebuild, a.status)) return;
+    if (!forced && !building(a)) return;
     for (std::int64_t slot = static_cast<std::int64_t>(launch.block) * blockDim.x + threadIdx.x;
          slot < a.num_atoms; slot += static_cast<std::int64_t>(launch.blocks) * blockDim.x)
     {
@@ -1214,7 +1223,7 @@ template <typename T>
 __device__ __forceinline__ void md_halo_body(const StepArgs<T>& a, const Launch launch,
                                              int forced)
 {
-    if (!forced && !rebuilding(a.rebuild, a.status)) return;
+    if (!forced && !building(a)) return;
     const int lane = lane_id();
     const index_t dims[3] = {a.nx, a.ny, a.nz};
     const std::int64_t waves = static_cast<std::int64_t>(launch.blocks) * (blockDim.x / kWave);
@@ -1377,7 +1386,7 @@ __device__ __forceinline__ void md_scan_body(const StepArgs<T>& a, const Launch 
 template <typename T>
 __global__ void __launch_bounds__(kListScanThreads) md_scan_kernel(StepArgs<T> a, int forced)
 {
-    if (!forced && !rebuilding(a.rebuild, a.status)) return;
+    if (!forced && !building(a)) return;
     md_scan_body(a, own_launch());
 }
 
@@ -1401,47 +1410,128 @@ __global__ void __launch_bounds__(kBlock) md_scatter_halo_kernel(StepArgs<T> a,
     md_scatter_halo_body(a, own_launch(), scatter_blocks, forced);
 }
 
-// Systems of at most kSmallBuild atoms: the whole build (assign, scan, scatter with the halo
-// listing, order, unpack, fill) by one block of 1,024 threads, its phases separated by the
-// block's barriers instead of kernel boundaries: one launch on every step where the build takes
-// six. The gate is read once per phase by one thread (a phase may set a status bit, and the
-// phases after it then do nothing, as the launches of a large build do); every phase is the same
-// body the large build runs, so the list is the same bit for bit.
-constexpr std::int64_t kSmallBuild = 2048;
-
+// The sort of a build by one block with the sub-bins' counts in LDS: each atom's sub-bin, the
+// counts' prefix sums (bin_offsets) and the atoms by sub-bin in any order within one (`unordered`,
+// which md_order_body ranks by id). What the assign, scan and scatter launches do for a large
+// system, in one launch: on nearly every step these are idle, and each dependent launch costs a
+// captured step 1.5 to 2 us. `counts` holds bins + 1 zeros; kInFlight positions are read before
+// any is used (bound by the latency of one block's reads: 13 us at 10,007 atoms, 27 at 32,768).
 template <typename T>
-__global__ void __launch_bounds__(kListScanThreads) md_build_small_kernel(StepArgs<T> a, T radius,
-                                                                          T cull_squared,
-                                                                          int forced)
+__device__ __forceinline__ void md_sort_body(const StepArgs<T>& a, index_t* counts)
+{
+    __shared__ index_t shared[kListScanWaves];
+    constexpr int kInFlight = 4;
+    const std::int64_t n = a.num_atoms;
+    const T wx = a.grid_widths[0], wy = a.grid_widths[1], wz = a.grid_widths[2];
+    for (std::int64_t base = threadIdx.x; base < n; base += kInFlight * kListScanThreads)
+    {
+        T x[kInFlight][3];
+#pragma unroll
+        for (int k = 0; k < kInFlight; ++k)
+        {
+            const std::int64_t slot = base + k * kListScanThreads;
+            const T* p = a.positions + 3 * (slot < n ? slot : 0);
+            for (int c = 0; c < 3; ++c) x[k][c] = p[c];
+        }
+#pragma unroll
+        for (int k = 0; k < kInFlight; ++k)
+        {
+            const std::int64_t slot = base + k * kListScanThreads;
+            if (slot >= n) continue;
+            const index_t bin = static_cast<index_t>(
+                sub_bin(x[k][0], wx, a.nx) + row_first_bin(sub_bin(x[k][1], wy, a.ny),
+                                                           sub_bin(x[k][2], wz, a.nz), a.nx, a.ny,
+                                                           a.nz));
+            a.bin_of[slot] = bin;
+            atomicAdd(counts + bin, 1);
+        }
+    }
+    __syncthreads();
+    // a run of counts per thread, an odd number of them so that the threads' reads spread over
+    // the banks
+    const index_t total_bins = static_cast<index_t>(a.bins) + 1;
+    const index_t per = ((total_bins + kListScanThreads - 1) / kListScanThreads) | 1;
+    const index_t from = static_cast<index_t>(threadIdx.x) * per;
+    const index_t to = from + per < total_bins ? from + per : total_bins;
+    index_t sum = 0;
+    for (index_t k = from; k < to; ++k) sum += counts[k];
+    index_t total;
+    index_t running = block_exclusive_sum(sum, shared, &total);
+    for (index_t k = from; k < to; ++k)
+    {
+        const index_t count = counts[k];
+        counts[k] = running;
+        running += count;
+    }
+    __syncthreads();
+    for (index_t k = threadIdx.x; k < total_bins; k += kListScanThreads)
+        a.bin_offsets[k] = counts[k];
+    __syncthreads();
+    // each atom takes the next place of its sub-bin
+    for (std::int64_t base = threadIdx.x; base < n; base += kInFlight * kListScanThreads)
+    {
+        index_t bin[kInFlight];
+#pragma unroll
+        for (int k = 0; k < kInFlight; ++k)
+        {
+            const std::int64_t slot = base + k * kListScanThreads;
+            bin[k] = slot < n ? a.bin_of[slot] : -1;
+        }
+#pragma unroll
+        for (int k = 0; k < kInFlight; ++k)
+            if (bin[k] >= 0)
+                a.unordered[atomicAdd(counts + bin[k], 1)] =
+                    static_cast<index_t>(base + k * kListScanThreads);
+    }
+}
+
+// Bytes of dynamic LDS of the one-block sort.
+inline std::size_t sort_bytes(std::int64_t bins)
+{
+    return static_cast<std::size_t>(bins + 1) * sizeof(index_t);
+}
+
+// The sort; with kWhole everything but the fill (the order with the halo listing, then the
+// frame home), its phases separated by the block's barriers instead of kernel boundaries. The
+// gate is read once per phase by one thread (a phase may set a status bit, and the phases after
+// it then do nothing, as the launches of a large build do); the bodies are those a large build
+// runs, so the list is the same bit for bit.
+template <typename T, bool kWhole>
+__global__ void __launch_bounds__(kListScanThreads) md_sort_kernel(StepArgs<T> a, int forced)
 {
     __shared__ int open;
-    const Launch one{0, 1};
+    extern __shared__ __align__(16) unsigned char dynamic_shared[];
+    index_t* counts = reinterpret_cast<index_t*>(dynamic_shared);
+    if (!forced && !building(a)) return;
+    for (index_t k = threadIdx.x; k <= a.bins; k += kListScanThreads) counts[k] = 0;
+    __syncthreads();
+    md_sort_body(a, counts);
+    if (!kWhole) return;
     auto gate = [&]() {
-        if (threadIdx.x == 0) open = forced || rebuilding(a.rebuild, a.status);
         __syncthreads();
-        const bool go = open != 0;
-        // before thread 0 reads the gate again
+        if (threadIdx.x == 0) open = forced || building(a);
         __syncthreads();
-        return go;
+        return open != 0;
     };
-    if (!gate()) return;
-    md_assign_body(a, one, 1);
-    __syncthreads();
-    if (!gate()) return;
-    md_scan_body(a, Launch{0, 1});
-    __syncthreads();
-    if (!gate()) return;
-    md_scatter_body(a, one, 1);
-    md_halo_body(a, one, 1);
-    __syncthreads();
+    const Launch one{0, 1};
     if (!gate()) return;
     md_order_body(a, one, 1);
-    __syncthreads();
+    md_halo_body(a, one, 1);
     if (!gate()) return;
     md_unpack_body(a, one, 1);
-    __syncthreads();
-    if (!gate()) return;
-    md_fill_body(a, one, radius, cull_squared, 1);
+}
+
+// The order and the halo listing, both after the sort, in one launch: the first `order_blocks`
+// blocks order, the rest list the halos.
+template <typename T>
+__global__ void __launch_bounds__(kBlock) md_order_halo_kernel(StepArgs<T> a,
+                                                               index_t order_blocks, int forced)
+{
+    const Launch launch = own_launch();
+    if (launch.block < order_blocks)
+        md_order_body(a, Launch{launch.block, order_blocks}, forced);
+    else
+        md_halo_body(a, Launch{launch.block - order_blocks, launch.blocks - order_blocks}, forced);
 }
 
 // The periodic frame of a brick. Along each axis every position p is replaced by its image nearest
@@ -1543,7 +1633,7 @@ __device__ __forceinline__ void md_fill_body(const StepArgs<T>& a, const Launch 
 {
 #pragma clang fp contract(off)
     using V4 = typename Vec4<T>::type;
-    if (!forced && !rebuilding(a.rebuild, a.status)) return;
+    if (!forced && !building(a)) return;
     const T radius_squared = radius * radius;
     const int lane = lane_id();
     const V4* pos = reinterpret_cast<const V4*>(a.positions4);
@@ -2742,6 +2832,29 @@ inline unsigned gated_grid(std::int64_t items, int per_block = kBlock)
         std::max<std::int64_t>(1, std::min<std::int64_t>(blocks_for(items, per_block), kGatedBlocks)));
 }
 
+// Kernels taking more than 64 KiB of dynamic LDS say so before their launch (a refusal shows
+// as the launch's own error).
+template <typename Kernel>
+void allow_shared(Kernel kernel, std::size_t bytes)
+{
+    if (bytes > 65536)
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                  hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  static_cast<int>(bytes));
+}
+
+// Systems whose build sorts in one block (md_sort_kernel), with its counts in the LDS of a block;
+// up to kWholeSort atoms the block also orders, lists the halos and puts the frame home. A step
+// (argon, skin 0.1 nm, a build every 16 to 21 steps) with separate launches / the sort in one /
+// everything but the fill in one: 512 atoms 25.2 / 23.7 / 20.8 us, 1,000 25.6 / 23.7 / 21.7,
+// 2,000 26.1 / 22.6 / 24.0, 4,096 27.3 / 24.0 / 29.2, 32,768 34.7 / 32.5 / -, 100,000 (skin 0.2)
+// 51.0 / 49.5 / - and (skin 0.1) 47.1 / 47.8 / -: past some 65,536 atoms the one block's sort
+// costs a build what the launches cost the steps between. (One block that also filled took 36 us
+// at 512 atoms and 55 at 2,000.)
+constexpr std::int64_t kWholeSort = 1024;
+constexpr std::int64_t kOneBlockSort = 65536;
+constexpr std::size_t kSortBytes = 144 * 1024;
+
 template <typename T>
 int launch_md_rebuild(const StepArgs<T>& a, double radius, int forced, hipStream_t stream)
 {
@@ -2749,10 +2862,31 @@ int launch_md_rebuild(const StepArgs<T>& a, double radius, int forced, hipStream
     const T r = static_cast<T>(radius);
     // culling keeps every sub-bin a pair within R could sit in, with room for rounding
     const T cull = static_cast<T>(radius * (1.0 + 1e-4) + 1e-6);
-    if (n <= kSmallBuild)
+    if (n <= kWholeSort && sort_bytes(a.bins) <= kSortBytes)
     {
-        md_build_small_kernel<T><<<1, kListScanThreads, 0, stream>>>(a, r, cull * cull, forced);
-        NDN_LAUNCHED("md_build_small");
+        allow_shared(md_sort_kernel<T, true>, sort_bytes(a.bins));
+        md_sort_kernel<T, true><<<1, kListScanThreads, sort_bytes(a.bins), stream>>>(a, forced);
+        NDN_LAUNCHED("md_sort");
+        md_unpack_fill_kernel<T><<<gated_grid(a.bins, kBlock / kWave), kBlock, 0, stream>>>(
+            a, 0, r, cull * cull, forced);
+        NDN_LAUNCHED("md_fill");
+        return NDN_OK;
+    }
+    if (n <= kOneBlockSort && sort_bytes(a.bins) <= kSortBytes)
+    {
+        allow_shared(md_sort_kernel<T, false>, sort_bytes(a.bins));
+        md_sort_kernel<T, false><<<1, kListScanThreads, sort_bytes(a.bins), stream>>>(a, forced);
+        NDN_LAUNCHED("md_sort");
+        const unsigned order = gated_grid(n);
+        const unsigned halo = gated_grid(a.bricks, kBlock / kWave);
+        md_order_halo_kernel<T><<<order + halo, kBlock, 0, stream>>>(
+            a, static_cast<index_t>(order), forced);
+        NDN_LAUNCHED("md_order_halo");
+        const unsigned unpack = gated_grid(n);
+        const unsigned fill = gated_grid(a.bins, kBlock / kWave);
+        md_unpack_fill_kernel<T><<<unpack + fill, kBlock, 0, stream>>>(
+            a, static_cast<index_t>(unpack), r, cull * cull, forced);
+        NDN_LAUNCHED("md_unpack_fill");
         return NDN_OK;
     }
     md_assign_kernel<T><<<gated_grid(n), kBlock, 0, stream>>>(a, forced);
@@ -2802,17 +2936,6 @@ std::size_t max_block_bytes()
         hipSuccess)
         return 65536;
     return static_cast<std::size_t>(std::max(per_block, 65536));
-}
-
-// Kernels taking more than 64 KiB of dynamic LDS say so before their launch (a refusal shows
-// as the launch's own error).
-template <typename Kernel>
-void allow_shared(Kernel kernel, std::size_t bytes)
-{
-    if (bytes > 65536)
-        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
-                                  hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  static_cast<int>(bytes));
 }
 
 // The force launch of one schedule.
@@ -3329,7 +3452,7 @@ __global__ void __launch_bounds__(kListScanThreads) batch_scan_kernel(BatchTable
     if (!batch_builds(t)) return;
     const BatchBlock b = batch_block(t.map, t.blocks, kPartScan);
     const StepArgs<T> a = t.members[b.member].a;
-    if (!rebuilding(a.rebuild, a.status)) return;
+    if (!building(a)) return;
     md_scan_body(a, b.launch);
 }
 

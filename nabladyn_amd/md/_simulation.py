@@ -112,10 +112,22 @@ _BRICKS = ((4, 4, 8), (4, 2, 8), (2, 2, 8), (2, 2, 4), (2, 1, 4), (1, 1, 4), (1,
            (1, 1, 1))
 
 
+# A force launch of fewer blocks leaves compute units idle: a step of 4,096 / 13,824 / 32,768 argon
+# atoms (skin 0.1 nm) took 42 / 41 / 40 us at 18 / 32 / 108 bricks of 4 x 4 x 8 sub-bins, and 27 /
+# 28 / 34 us at 150 / 256 / 198 smaller ones; at 300 / 480 / 363 still smaller ones 29 / 29 / 35.
+_FILLING_BRICKS = 150
+
+
+def _brick_count(shape, dims) -> int:
+    return math.prod(-(-d // b) for d, b in zip(dims, shape))
+
+
 def brick_shapes(dims: list[int], num_atoms: int, dtype: torch.dtype, reserve: int = 0):
     """The brick shapes worth trying for this grid, largest first: those whose expected halo
     (atoms per sub-bin times its sub-bins, with a tenth to spare) fits the LDS budget less
-    `reserve` positions' worth kept for the potential."""
+    `reserve` positions' worth kept for the potential, from the largest that gives the force
+    launch a block for most of the chip's 256 compute units (``_FILLING_BRICKS``; down to 8
+    sub-bins a brick, below which staging the halos costs more than more blocks save)."""
     per_bin = num_atoms / math.prod(dims)
     limit = halo_limit(dtype) - reserve
     shapes = []
@@ -123,6 +135,9 @@ def brick_shapes(dims: list[int], num_atoms: int, dtype: torch.dtype, reserve: i
         halo = math.prod(min(b + 4, d) for b, d in zip(shape, dims))
         if 1.1 * halo * per_bin <= limit:
             shapes.append(shape)
+    while (len(shapes) > 1 and math.prod(shapes[1]) >= 8
+           and _brick_count(shapes[0], dims) < _FILLING_BRICKS):
+        shapes.pop(0)
     return shapes or [_BRICKS[-1]]
 
 
@@ -244,7 +259,7 @@ class _MDNeighbors:
     def set_bricks(self, shape) -> None:
         """Bricks of `shape` sub-bins; their halos unsized until `size_halo`."""
         device = self.buffers["counts"].device
-        bricks = math.prod(-(-d // b) for d, b in zip(self.dims, shape))
+        bricks = _brick_count(shape, self.dims)
         self.brick = tuple(shape)
         self.bricks = bricks
         self.buffers["halo_runs"] = torch.zeros(bricks * _HALO_RUNS, dtype=torch.int32, device=device)
