@@ -17,6 +17,7 @@
 
 #include <algorithm>
 #include <climits>
+#include <type_traits>
 
 #include "common.hpp"
 #include "pair_forces.hpp"
@@ -75,6 +76,116 @@ __global__ void zero_kernel(T* __restrict__ data, std::int64_t count)
         data[i] = T(0);
 }
 
+// ---- a one-type table in LDS ----------------------------------------------------------------
+
+// A table of one type whose segments' cubics each block writes into LDS: u = u1 + s(A + s(B + s C)),
+// du/dt = A + s(2B + 3 s C). A pair then reads one 4-vector instead of gathering four knots from
+// memory (a table's knots were as many gathers as its neighbors' positions) and forming the
+// cubic, and the knot coordinate's division is a product corrected by its remainder. E, F and W
+// of 205,875 atoms (152 entries a row) 222 -> 198 us a call; 50,653 atoms in fp64 (193) 151 -> 126.
+template <typename T>
+struct StagedTable
+{
+    using V4 = typename std::conditional<sizeof(T) == 4, float4, double4>::type;
+    static constexpr bool kStaged = true;
+    const T* __restrict__ padded;  // [K + 2]
+    const T* __restrict__ start;
+    const T* __restrict__ spacing;
+    int knots;
+    // set by the block
+    const V4* segments;
+    T first, step, inverse_step;
+
+    __device__ __forceinline__ void stage(unsigned char* lds)
+    {
+        V4* out = reinterpret_cast<V4*>(lds);
+        for (int k = threadIdx.x; k < knots - 1; k += blockDim.x)
+        {
+            const T u0 = padded[k], u1 = padded[k + 1], u2 = padded[k + 2], u3 = padded[k + 3];
+            V4 c;
+            c.x = u1;
+            c.y = T(0.5) * (u2 - u0);
+            c.z = T(0.5) * (T(2) * u0 - T(5) * u1 + T(4) * u2 - u3);
+            c.w = T(0.5) * (T(3) * (u1 - u2) + u3 - u0);
+            out[k] = c;
+        }
+        segments = out;
+        first = start[0];
+        step = spacing[0];
+        inverse_step = T(1) / step;
+        __syncthreads();
+    }
+
+    __device__ __forceinline__ int row(std::int64_t, std::int64_t) const
+    {
+        return 0;
+    }
+
+    __device__ __forceinline__ void eval(int, T r2, T& u, T& fs) const
+    {
+        const T r = pair_distance(r2);
+        const T offset = r - first;
+        const T q = offset * inverse_step;
+        const T x = fma(fma(-q, step, offset), inverse_step, q);
+        T segment = floor(x);
+        segment = segment < T(0) ? T(0) : (segment > T(knots - 2) ? T(knots - 2) : segment);
+        const T t = x - segment;
+        const V4 c = segments[static_cast<int>(segment)];
+        const T s = t > T(0) ? t : T(0);
+        // below the first knot s is 0 and the tangent remains
+        u = c.x + s * (c.y + s * (c.z + s * c.w)) + c.y * (t - s);
+        const T du_dt = c.y + s * (T(2) * c.z + T(3) * s * c.w);
+        fs = -(du_dt * inverse_step) * refined_reciprocal(r);
+    }
+};
+
+template <class Pot, typename = void>
+struct IsStaged : std::false_type
+{
+};
+template <class Pot>
+struct IsStaged<Pot, std::enable_if_t<Pot::kStaged>> : std::true_type
+{
+};
+
+// The LDS a block may give a staged table: eight blocks of it share a compute unit.
+constexpr std::size_t kStagedBytes = 16384;
+
+template <typename T>
+bool stages(const PotentialView<T>& view)
+{
+    return view.kind == NDN_TABLE && view.table.num_types == 1 &&
+           (static_cast<std::size_t>(view.table.knots) - 1) * 4 * sizeof(T) <= kStagedBytes;
+}
+
+template <typename T>
+StagedTable<T> staged_table(const Table<T>& table)
+{
+    StagedTable<T> staged{};
+    staged.padded = table.padded;
+    staged.start = table.start;
+    staged.spacing = table.spacing;
+    staged.knots = table.knots;
+    return staged;
+}
+
+template <class Pot>
+std::size_t staged_bytes(const Pot&)
+{
+    return 0;
+}
+template <typename T>
+std::size_t staged_bytes(const StagedTable<T>& pot)
+{
+    return (static_cast<std::size_t>(pot.knots) - 1) * 4 * sizeof(T);
+}
+
+template <class Pot>
+__device__ __forceinline__ void stage_in_block(Pot& pot, unsigned char* lds)
+{
+    if constexpr (IsStaged<Pot>::value) pot.stage(lds);
+}
+
 // ---- half-list schedule ---------------------------------------------------------------------
 
 // The sum of `value` over each run of lanes with the same key (a run starts where the key
@@ -102,6 +213,8 @@ __global__ void __launch_bounds__(kBlock) half_list_kernel(
     T cutoff_squared, Pot pot, T* __restrict__ forces, double* __restrict__ partials)
 {
     __shared__ double shared[16];
+    extern __shared__ __align__(16) unsigned char staged[];
+    stage_in_block(pot, staged);
     const std::int64_t frame = blockIdx.y;
     positions += 3 * frame * num_atoms;
     cell += 3 * frame;
@@ -215,8 +328,11 @@ constexpr int full_rows_ahead()
     return sizeof(T) == 4 ? 8 : 4;
 }
 
-template <typename T, class Pot, bool kForces, bool kVirial>
-__global__ void __launch_bounds__(kBlock) full_rows_kernel(
+// kSplit waves share a slice, each taking every kSplit-th turn of its rows, and their forces are
+// added in wave order through LDS: a small system's slices are too few waves for the chip (a wave
+// per slice took 27 us for 864 atoms, 14 waves walking 150 entries one turn after another).
+template <typename T, class Pot, bool kForces, bool kVirial, int kSplit>
+__global__ void __launch_bounds__(kSplit > 4 ? kSplit * kWave : kBlock) full_rows_kernel(
     const T* __restrict__ positions, const T* __restrict__ cell, const index_t* __restrict__ rows,
     const index_t* __restrict__ counts, const index_t* __restrict__ slices,
     const index_t* __restrict__ index, std::int64_t capacity, index_t num_atoms,
@@ -224,6 +340,8 @@ __global__ void __launch_bounds__(kBlock) full_rows_kernel(
 {
     constexpr int kAhead = full_rows_ahead<T, Pot>();
     __shared__ double shared[16];
+    extern __shared__ __align__(16) unsigned char staged[];
+    stage_in_block(pot, staged);
     const std::int64_t slices_total = (static_cast<std::int64_t>(num_atoms) + kWave - 1) / kWave;
     // frames of one system (blockIdx.y): each frame's arrays follow the previous frame's (rows
     // [N], counts [N], slices [N / 64 + 1], `capacity` index entries)
@@ -242,10 +360,13 @@ __global__ void __launch_bounds__(kBlock) full_rows_kernel(
     const int lane = lane_id();
     T energy = 0;
     T w[6] = {0, 0, 0, 0, 0, 0};
-    const std::int64_t waves = static_cast<std::int64_t>(gridDim.x) * (blockDim.x / kWave);
-    for (std::int64_t slice =
-             static_cast<std::int64_t>(blockIdx.x) * (blockDim.x / kWave) + threadIdx.x / kWave;
-         slice < slices_total; slice += waves)
+    __shared__ T split_forces[kForces && kSplit > 1 ? kSplit * kWave * 3 : 1];
+    const int wave = threadIdx.x / kWave;
+    const int share = wave % kSplit;
+    const int together = blockDim.x / kWave / kSplit;  // slices a block walks at a time
+    const std::int64_t stride = static_cast<std::int64_t>(gridDim.x) * together;
+    for (std::int64_t slice = static_cast<std::int64_t>(blockIdx.x) * together + wave / kSplit;
+         slice < slices_total; slice += stride)
     {
         const std::int64_t row = slice * kWave + lane;
         const bool live = row < num_atoms;
@@ -264,7 +385,7 @@ __global__ void __launch_bounds__(kBlock) full_rows_kernel(
         const T* p = positions + 3LL * me;
         const T px = p[0], py = p[1], pz = p[2];
         T fx = 0, fy = 0, fz = 0;
-        for (std::int64_t k0 = 0; ballot(k0 < walk) != 0; k0 += kAhead)
+        for (std::int64_t k0 = share * kAhead; ballot(k0 < walk) != 0; k0 += kSplit * kAhead)
         {
             index_t j[kAhead];
 #pragma unroll
@@ -312,7 +433,25 @@ __global__ void __launch_bounds__(kBlock) full_rows_kernel(
                 }
             }
         }
-        if (kForces && own)
+        if (kForces && kSplit > 1)
+        {
+            // one slice a block: every wave reaches these barriers equally often
+            T* mine = split_forces + 3 * (share * kWave + lane);
+            mine[0] = fx;
+            mine[1] = fy;
+            mine[2] = fz;
+            __syncthreads();
+            if (share == 0)
+                for (int w = 1; w < kSplit; ++w)
+                {
+                    const T* theirs = split_forces + 3 * (w * kWave + lane);
+                    fx += theirs[0];
+                    fy += theirs[1];
+                    fz += theirs[2];
+                }
+            __syncthreads();
+        }
+        if (kForces && own && share == 0)
         {
             forces[3LL * i] = fx;
             forces[3LL * i + 1] = fy;
@@ -466,50 +605,88 @@ void launch_half(const T* x, const T* cell, const index_t* pairs, std::int64_t c
 {
     const dim3 blocks(static_cast<unsigned>(columns_blocks), static_cast<unsigned>(frames));
     if (forces && virial)
-        half_list_kernel<T, Pot, true, true><<<blocks, kBlock, 0, stream>>>(
+        half_list_kernel<T, Pot, true, true><<<blocks, kBlock, staged_bytes(pot), stream>>>(
             x, cell, pairs, capacity, num_atoms, cutoff_squared, pot, forces, partials);
     else if (forces)
-        half_list_kernel<T, Pot, true, false><<<blocks, kBlock, 0, stream>>>(
+        half_list_kernel<T, Pot, true, false><<<blocks, kBlock, staged_bytes(pot), stream>>>(
             x, cell, pairs, capacity, num_atoms, cutoff_squared, pot, forces, partials);
     else if (virial)
-        half_list_kernel<T, Pot, false, true><<<blocks, kBlock, 0, stream>>>(
+        half_list_kernel<T, Pot, false, true><<<blocks, kBlock, staged_bytes(pot), stream>>>(
             x, cell, pairs, capacity, num_atoms, cutoff_squared, pot, forces, partials);
     else
-        half_list_kernel<T, Pot, false, false><<<blocks, kBlock, 0, stream>>>(
+        half_list_kernel<T, Pot, false, false><<<blocks, kBlock, staged_bytes(pot), stream>>>(
             x, cell, pairs, capacity, num_atoms, cutoff_squared, pot, forces, partials);
+}
+
+// Waves that share a slice, by the slices of the launch. One where the slices fill the chip by
+// themselves (2,097,152 atoms in lattice order: 646 us against 702 with four, whose last turns
+// are partly empty). Four below 4,096 slices: 205,875 atoms of a table in arbitrary order 198 ->
+// 160 us (the four waves meet the same neighbors, and share their lines), 50,653 in fp64 125 ->
+// 111, 120,000 LJ atoms in lattice order 94 -> 89. Sixteen below 128 slices, a wave per 64 of
+// whose rows are too few to hide any latency.
+int full_split(std::int64_t num_atoms, std::int64_t frames)
+{
+    const std::int64_t slices = (num_atoms + kWave - 1) / kWave * frames;
+    return slices >= 4096 ? 1 : (slices >= 128 ? 4 : 16);
+}
+
+// Blocks of the full-row launch over each of `frames` frames: a wave (or a block of `split` waves)
+// per 64 rows, at most kHalfBlocks blocks striding, and no more than the partial slots that every
+// workspace holds (kPartialSlots, and half_blocks(N) of each frame).
+int full_blocks(std::int64_t num_atoms, std::int64_t frames, int split)
+{
+    const std::int64_t slices = (num_atoms + kWave - 1) / kWave;
+    const std::int64_t together = split == 1 ? kBlock / kWave : 1;
+    const std::int64_t blocks = (slices + together - 1) / together;
+    const std::int64_t slots = std::max<std::int64_t>(half_blocks(num_atoms), kPartialSlots / frames);
+    return static_cast<int>(
+        std::max<std::int64_t>(1, std::min<std::int64_t>({blocks, kHalfBlocks, slots})));
+}
+
+template <typename T, class Pot, int kSplit>
+void launch_full_split(const T* x, const T* cell, const index_t* rows, const index_t* counts,
+                       const index_t* slices, const index_t* index, std::int64_t capacity,
+                       index_t num_atoms, T cutoff_squared, const Pot& pot, T* forces, bool virial,
+                       double* partials, const dim3& blocks, hipStream_t stream)
+{
+    constexpr int kThreads = kSplit > 4 ? kSplit * kWave : kBlock;
+    const std::size_t lds = staged_bytes(pot);
+    if (forces && virial)
+        full_rows_kernel<T, Pot, true, true, kSplit><<<blocks, kThreads, lds, stream>>>(
+            x, cell, rows, counts, slices, index, capacity, num_atoms, cutoff_squared, pot,
+            forces, partials);
+    else if (forces)
+        full_rows_kernel<T, Pot, true, false, kSplit><<<blocks, kThreads, lds, stream>>>(
+            x, cell, rows, counts, slices, index, capacity, num_atoms, cutoff_squared, pot,
+            forces, partials);
+    else if (virial)
+        full_rows_kernel<T, Pot, false, true, kSplit><<<blocks, kThreads, lds, stream>>>(
+            x, cell, rows, counts, slices, index, capacity, num_atoms, cutoff_squared, pot,
+            forces, partials);
+    else
+        full_rows_kernel<T, Pot, false, false, kSplit><<<blocks, kThreads, lds, stream>>>(
+            x, cell, rows, counts, slices, index, capacity, num_atoms, cutoff_squared, pot,
+            forces, partials);
 }
 
 template <typename T, class Pot>
 void launch_full(const T* x, const T* cell, const index_t* rows, const index_t* counts,
                  const index_t* slices, const index_t* index, std::int64_t capacity,
                  index_t num_atoms, T cutoff_squared, const Pot& pot, T* forces, bool virial,
-                 double* partials, int row_blocks, hipStream_t stream, int frames = 1)
+                 double* partials, hipStream_t stream, int frames = 1)
 {
-    const dim3 blocks(static_cast<unsigned>(row_blocks), static_cast<unsigned>(frames));
-    if (forces && virial)
-        full_rows_kernel<T, Pot, true, true><<<blocks, kBlock, 0, stream>>>(
-            x, cell, rows, counts, slices, index, capacity, num_atoms, cutoff_squared, pot,
-            forces, partials);
-    else if (forces)
-        full_rows_kernel<T, Pot, true, false><<<blocks, kBlock, 0, stream>>>(
-            x, cell, rows, counts, slices, index, capacity, num_atoms, cutoff_squared, pot,
-            forces, partials);
-    else if (virial)
-        full_rows_kernel<T, Pot, false, true><<<blocks, kBlock, 0, stream>>>(
-            x, cell, rows, counts, slices, index, capacity, num_atoms, cutoff_squared, pot,
-            forces, partials);
+    const int split = full_split(num_atoms, frames);
+    const dim3 blocks(static_cast<unsigned>(full_blocks(num_atoms, frames, split)),
+                      static_cast<unsigned>(frames));
+    if (split == 1)
+        launch_full_split<T, Pot, 1>(x, cell, rows, counts, slices, index, capacity, num_atoms,
+                                     cutoff_squared, pot, forces, virial, partials, blocks, stream);
+    else if (split == 4)
+        launch_full_split<T, Pot, 4>(x, cell, rows, counts, slices, index, capacity, num_atoms,
+                                     cutoff_squared, pot, forces, virial, partials, blocks, stream);
     else
-        full_rows_kernel<T, Pot, false, false><<<blocks, kBlock, 0, stream>>>(
-            x, cell, rows, counts, slices, index, capacity, num_atoms, cutoff_squared, pot,
-            forces, partials);
-}
-
-// Blocks of the full-row launch: a wave per 64 rows, at most kHalfBlocks blocks striding.
-int full_blocks(std::int64_t num_atoms)
-{
-    const std::int64_t slices = (num_atoms + kWave - 1) / kWave;
-    const std::int64_t blocks = (slices + kBlock / kWave - 1) / (kBlock / kWave);
-    return static_cast<int>(std::max<std::int64_t>(1, std::min<std::int64_t>(blocks, kHalfBlocks)));
+        launch_full_split<T, Pot, 16>(x, cell, rows, counts, slices, index, capacity, num_atoms,
+                                      cutoff_squared, pot, forces, virial, partials, blocks, stream);
 }
 
 template <typename T>
@@ -522,7 +699,7 @@ int pair_efw_full_impl(const void* positions, const void* cell, std::int64_t num
     PotentialView<T> view;
     const int prepared = prepare_potential<T>(pot, workspace, stream, &view);
     if (prepared != NDN_OK) return prepared;
-    const int blocks = full_blocks(num_atoms);
+    const int blocks = full_blocks(num_atoms, 1, full_split(num_atoms, 1));
     auto* partials = reinterpret_cast<double*>(static_cast<std::uint8_t*>(workspace) +
                                                coefficient_bytes(pot, sizeof(T)));
     T* f = static_cast<T*>(forces);
@@ -531,10 +708,13 @@ int pair_efw_full_impl(const void* positions, const void* cell, std::int64_t num
     const index_t n = static_cast<index_t>(num_atoms);
     if (view.kind == NDN_LJ)
         launch_full<T>(x, L, rows, counts, slices, index, capacity, n, view.cutoff_squared,
-                       view.lj, f, virial != nullptr, partials, blocks, stream);
+                       view.lj, f, virial != nullptr, partials, stream);
+    else if (stages(view))
+        launch_full<T>(x, L, rows, counts, slices, index, capacity, n, view.cutoff_squared,
+                       staged_table(view.table), f, virial != nullptr, partials, stream);
     else
         launch_full<T>(x, L, rows, counts, slices, index, capacity, n, view.cutoff_squared,
-                       view.table, f, virial != nullptr, partials, blocks, stream);
+                       view.table, f, virial != nullptr, partials, stream);
     NDN_LAUNCHED("full_rows");
     return finish<T>(partials, blocks, energy, virial, 1.0, stream);
 }
@@ -551,7 +731,7 @@ int pair_efw_full_frames_impl(const void* positions, const void* cells, std::int
     PotentialView<T> view;
     const int prepared = prepare_potential<T>(pot, workspace, stream, &view);
     if (prepared != NDN_OK) return prepared;
-    const int blocks = full_blocks(num_atoms);
+    const int blocks = full_blocks(num_atoms, frames, full_split(num_atoms, frames));
     auto* partials = reinterpret_cast<double*>(static_cast<std::uint8_t*>(workspace) +
                                                coefficient_bytes(pot, sizeof(T)));
     T* f = static_cast<T*>(forces);
@@ -561,10 +741,13 @@ int pair_efw_full_frames_impl(const void* positions, const void* cells, std::int
     const int count = static_cast<int>(frames);
     if (view.kind == NDN_LJ)
         launch_full<T>(x, L, nullptr, counts, slices, index, capacity, n, view.cutoff_squared,
-                       view.lj, f, virial != nullptr, partials, blocks, stream, count);
+                       view.lj, f, virial != nullptr, partials, stream, count);
+    else if (stages(view))
+        launch_full<T>(x, L, nullptr, counts, slices, index, capacity, n, view.cutoff_squared,
+                       staged_table(view.table), f, virial != nullptr, partials, stream, count);
     else
         launch_full<T>(x, L, nullptr, counts, slices, index, capacity, n, view.cutoff_squared,
-                       view.table, f, virial != nullptr, partials, blocks, stream, count);
+                       view.table, f, virial != nullptr, partials, stream, count);
     NDN_LAUNCHED("full_rows_frames");
     if (energy == nullptr && virial == nullptr) return NDN_OK;
     finish_kernel<T><<<count, kBlock, 0, stream>>>(partials, blocks, static_cast<T*>(energy),
@@ -596,6 +779,9 @@ int pair_efw_impl(const void* positions, const void* cell, std::int64_t num_atom
     if (view.kind == NDN_LJ)
         launch_half<T>(x, L, pairs, capacity, static_cast<index_t>(num_atoms), view.cutoff_squared,
                        view.lj, f, virial != nullptr, partials, blocks, stream);
+    else if (stages(view))
+        launch_half<T>(x, L, pairs, capacity, static_cast<index_t>(num_atoms), view.cutoff_squared,
+                       staged_table(view.table), f, virial != nullptr, partials, blocks, stream);
     else
         launch_half<T>(x, L, pairs, capacity, static_cast<index_t>(num_atoms), view.cutoff_squared,
                        view.table, f, virial != nullptr, partials, blocks, stream);
@@ -630,6 +816,9 @@ int pair_efw_frames_impl(const void* positions, const void* cells, std::int64_t 
     const int count = static_cast<int>(frames);
     if (view.kind == NDN_LJ)
         launch_half<T>(x, L, stacks, capacity, n, view.cutoff_squared, view.lj, f,
+                       virial != nullptr, partials, blocks, stream, count);
+    else if (stages(view))
+        launch_half<T>(x, L, stacks, capacity, n, view.cutoff_squared, staged_table(view.table), f,
                        virial != nullptr, partials, blocks, stream, count);
     else
         launch_half<T>(x, L, stacks, capacity, n, view.cutoff_squared, view.table, f,
