@@ -935,13 +935,20 @@ __global__ void __launch_bounds__(kBlock) fill_all_pairs_kernel(
 
 // The pair total and, above the capacity, the overflow bit with the pairs needed; then the
 // padding. Column k past the pairs holds (k mod N, k mod N) whatever the build, so after the
-// first frame only the columns between this total and the previous one need writing.
-__global__ void __launch_bounds__(kBlock) total_pad_kernel(
+// first frame only the columns between this total and the previous one need writing. A rebuild
+// that fits is committed in the same launch (reference_positions null for a first frame, whose
+// caller keeps the frame itself): its frame and cell become the reuse rule's reference. Every
+// block decides from the totals, which no block writes, so a status bit set meanwhile changes
+// nothing.
+template <typename T>
+__global__ void __launch_bounds__(kBlock) total_pad_commit_kernel(
     const index_t* __restrict__ pair_counts, const index_t* __restrict__ pair_offsets,
     index_t num_atoms, std::int64_t capacity, index_t* __restrict__ pair_total, index_t* status,
     index_t* __restrict__ pairs, const ListHeader* __restrict__ header, int first_frame,
     const index_t* __restrict__ full_slices, std::int64_t num_slices, std::int64_t full_capacity,
-    const index_t* rebuild)
+    const T* __restrict__ positions, const T* __restrict__ cell,
+    T* __restrict__ reference_positions, T* __restrict__ reference_cell,
+    index_t* __restrict__ rebuild_count, const index_t* rebuild)
 {
     if (!rebuilding(rebuild, status)) return;
     const index_t total = pair_offsets[num_atoms - 1] + pair_counts[num_atoms - 1];
@@ -969,19 +976,11 @@ __global__ void __launch_bounds__(kBlock) total_pad_kernel(
         pairs[column] = atom;
         pairs[capacity + column] = atom;
     }
-}
-
-template <typename T>
-__global__ void __launch_bounds__(kBlock) commit_rebuild_kernel(
-    const T* __restrict__ positions, const T* __restrict__ cell, index_t num_atoms,
-    T* __restrict__ reference_positions, T* __restrict__ reference_cell,
-    index_t* __restrict__ rebuild_count, const index_t* rebuild, const index_t* status)
-{
-    const std::int64_t index = static_cast<std::int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (index >= 3LL * num_atoms || !rebuilding(rebuild, status)) return;
-    reference_positions[index] = positions[index];
-    if (index < 3) reference_cell[index] = cell[index];
-    if (index == 0) ++rebuild_count[0];
+    if (reference_positions == nullptr) return;
+    for (std::int64_t k = gid; k < 3LL * num_atoms; k += stride)
+        reference_positions[k] = positions[k];
+    if (gid < 3) reference_cell[gid] = cell[gid];
+    if (gid == 0) ++rebuild_count[0];
 }
 
 template <typename T>
@@ -1140,22 +1139,21 @@ int launch_count(const T* positions, const T* cell, double radius, const ndn_nei
         launch_search<T, false>(cell, r2, b, rebuild, stream);
         NDN_LAUNCHED("count_pairs");
     }
-    int scanned = exclusive_scan(b.pair_counts, b.pair_offsets, b.num_atoms, b.scan_temp, rebuild,
-                                 b.status, stream);
-    if (scanned != NDN_OK) return scanned;
-    if (full)
-    {
-        // slices + 1 entries: the last (kept 0 by the counts) becomes the total.
-        scanned = exclusive_scan(b.full_slices, b.full_slices, slices + 1, b.scan_temp, rebuild,
-                                 b.status, stream);
-        if (scanned != NDN_OK) return scanned;
-    }
-    return NDN_OK;
+    // the columns' offsets, and with a full list the slices' (slices + 1 entries: the last, an
+    // output only, becomes the total), in the same launches; the slices' tile sums go where the
+    // build's unordered ids were
+    const ScanArray columns{b.pair_counts, b.pair_offsets, b.num_atoms,
+                            reinterpret_cast<index_t*>(b.scan_temp + kHeaderBytes)};
+    ScanArray widths{};
+    if (full) widths = ScanArray{b.full_slices, b.full_slices, slices + 1, b.unordered_ids};
+    return exclusive_scans(columns, widths, rebuild, b.status, stream);
 }
 
+// A first frame's (reference_positions null) or an update's fill, padding and commit.
 template <typename T>
-int launch_fill(const T* cell, double radius, const ndn_neighbor_buffers& b,
-                const index_t* rebuild, bool first_frame, hipStream_t stream)
+int launch_fill(const T* positions, const T* cell, double radius, const ndn_neighbor_buffers& b,
+                T* reference_positions, T* reference_cell, index_t* rebuild_count,
+                const index_t* rebuild, hipStream_t stream)
 {
     const index_t n = static_cast<index_t>(b.num_atoms);
     const T r = static_cast<T>(radius);
@@ -1182,11 +1180,12 @@ int launch_fill(const T* cell, double radius, const ndn_neighbor_buffers& b,
         launch_search<T, true>(cell, r2, b, rebuild, stream);
         NDN_LAUNCHED("fill_pairs");
     }
-    total_pad_kernel<<<kPadBlocks, kBlock, 0, stream>>>(
+    total_pad_commit_kernel<T><<<kPadBlocks, kBlock, 0, stream>>>(
         b.pair_counts, b.pair_offsets, n, b.capacity, b.pair_total, b.status, b.pairs,
-        reinterpret_cast<const ListHeader*>(b.scan_temp), first_frame ? 1 : 0,
-        full ? b.full_slices : nullptr, slices, b.full_capacity, rebuild);
-    NDN_LAUNCHED("total_pad");
+        reinterpret_cast<const ListHeader*>(b.scan_temp), reference_positions == nullptr ? 1 : 0,
+        full ? b.full_slices : nullptr, slices, b.full_capacity, positions, cell,
+        reference_positions, reference_cell, rebuild_count, rebuild);
+    NDN_LAUNCHED("total_pad_commit");
     return NDN_OK;
 }
 
@@ -1195,20 +1194,15 @@ int launch_rebuild(const T* positions, const T* cell, double radius, const ndn_n
                    T* reference_positions, T* reference_cell, index_t* rebuild_count,
                    const index_t* rebuild, hipStream_t stream)
 {
-    const index_t n = static_cast<index_t>(b.num_atoms);
     if (b.bits_words == 0)
     {
         const int grid = launch_grid<T>(positions, b, rebuild, stream);
         if (grid != NDN_OK) return grid;
     }
-    int step = launch_count<T>(positions, cell, radius, b, rebuild, stream);
-    if (step != NDN_OK) return step;
-    step = launch_fill<T>(cell, radius, b, rebuild, false, stream);
-    if (step != NDN_OK) return step;
-    commit_rebuild_kernel<T><<<blocks_for(3LL * n), kBlock, 0, stream>>>(
-        positions, cell, n, reference_positions, reference_cell, rebuild_count, rebuild, b.status);
-    NDN_LAUNCHED("commit_rebuild");
-    return NDN_OK;
+    const int counted = launch_count<T>(positions, cell, radius, b, rebuild, stream);
+    if (counted != NDN_OK) return counted;
+    return launch_fill<T>(positions, cell, radius, b, reference_positions, reference_cell,
+                          rebuild_count, rebuild, stream);
 }
 
 template int launch_rebuild<float>(const float*, const float*, double, const ndn_neighbor_buffers&,
@@ -1259,7 +1253,8 @@ template <typename T>
 int fill_first_frame_impl(const void* cell, double radius, const ndn_neighbor_buffers& b,
                           hipStream_t stream)
 {
-    return launch_fill<T>(static_cast<const T*>(cell), radius, b, nullptr, true, stream);
+    return launch_fill<T>(nullptr, static_cast<const T*>(cell), radius, b, nullptr, nullptr,
+                          nullptr, nullptr, stream);
 }
 
 template <typename T>

@@ -1,8 +1,13 @@
-// A gated exclusive scan of int32 values for the list builds: three launches (tile sums, one
-// block scanning the tile sums, tiles applied), each of which returns at once when the build
-// is not running, so a captured update pays three empty launches on steps without a rebuild.
-// The tile sums live after the list header in the caller's scan_temp buffer.
+// A gated exclusive scan of int32 values for the list builds, or of two arrays in the same
+// launches: tile sums, then tiles applied, each block first adding up the tile sums before its own
+// (integer sums: the same whatever the order). Past kScanOwnTiles tiles, where that would read
+// more than it saves, one block scans the tile sums in a launch between. Each launch returns at
+// once when the build is not running, so a captured update pays two empty launches on steps
+// without a rebuild. The first array's tile sums live after the list header in the caller's
+// scan_temp buffer, the second's in a scratch array of its own.
 #pragma once
+
+#include <algorithm>
 
 #include "common.hpp"
 
@@ -38,11 +43,19 @@ inline std::int64_t scan_bytes(std::int64_t items)
     return kHeaderBytes + 4 * (scan_tiles(items) + 1);
 }
 
-// The bodies take the block (a launch over a batch of systems passes each system's own).
-static __device__ __forceinline__ void scan_tile_sums_body(const index_t* __restrict__ input,
-                                                           std::int64_t count,
-                                                           index_t* __restrict__ tile_sums,
-                                                           index_t block)
+// Tiles up to which a block adds up the tile sums before its own: 16 reads a thread at most.
+constexpr std::int64_t kScanOwnTiles = 4096;
+
+// One array of a scan: `count` values, its tile sums (tiles of kScanTile).
+struct ScanArray
+{
+    const index_t* input;
+    index_t* output;  // may alias input: each block reads its whole tile before writing it
+    std::int64_t count;
+    index_t* tile_sums;
+};
+
+static __device__ __forceinline__ void scan_tile_sums_body(const ScanArray& a, index_t block)
 {
     __shared__ index_t shared[16];
     const std::int64_t base = static_cast<std::int64_t>(block) * kScanTile;
@@ -51,23 +64,30 @@ static __device__ __forceinline__ void scan_tile_sums_body(const index_t* __rest
     for (int k = 0; k < kScanPerThread; ++k)
     {
         const std::int64_t i = base + threadIdx.x + static_cast<std::int64_t>(k) * kBlock;
-        if (i < count) local += input[i];
+        if (i < a.count) local += a.input[i];
     }
     const index_t sum = block_sum(local, shared);
-    if (threadIdx.x == 0) tile_sums[block] = sum;
+    if (threadIdx.x == 0) a.tile_sums[block] = sum;
 }
 
+// The first `first_tiles` blocks take the first array, the rest the second.
 static __global__ void __launch_bounds__(kBlock) scan_tile_sums_kernel(
-    const index_t* __restrict__ input, std::int64_t count, index_t* __restrict__ tile_sums,
-    const index_t* rebuild, const index_t* status)
+    ScanArray first, ScanArray second, index_t first_tiles, const index_t* rebuild,
+    const index_t* status)
 {
     if (!rebuilding(rebuild, status)) return;
-    scan_tile_sums_body(input, count, tile_sums, static_cast<index_t>(blockIdx.x));
+    const index_t block = static_cast<index_t>(blockIdx.x);
+    if (block < first_tiles)
+        scan_tile_sums_body(first, block);
+    else
+        scan_tile_sums_body(second, block - first_tiles);
 }
 
-static __device__ __forceinline__ void scan_tile_prefix_body(index_t* __restrict__ tile_sums,
-                                                             std::int64_t tiles)
+static __global__ void __launch_bounds__(kBlock) scan_tile_prefix_kernel(
+    index_t* __restrict__ tile_sums, std::int64_t tiles, const index_t* rebuild,
+    const index_t* status)
 {
+    if (!rebuilding(rebuild, status)) return;
     __shared__ index_t shared[16];
     index_t carry = 0;
     for (std::int64_t base = 0; base < tiles; base += kScanTile)
@@ -95,20 +115,21 @@ static __device__ __forceinline__ void scan_tile_prefix_body(index_t* __restrict
     }
 }
 
-static __global__ void __launch_bounds__(kBlock) scan_tile_prefix_kernel(
-    index_t* __restrict__ tile_sums, std::int64_t tiles, const index_t* rebuild,
-    const index_t* status)
-{
-    if (!rebuilding(rebuild, status)) return;
-    scan_tile_prefix_body(tile_sums, tiles);
-}
-
-// out may alias in: each block reads its whole tile before writing it.
-static __device__ __forceinline__ void scan_apply_body(const index_t* input, std::int64_t count,
-                                                       const index_t* __restrict__ tile_prefix,
-                                                       index_t* output, index_t block)
+// kOwn: the tile sums are as they were summed and the block adds up those before its own; else
+// they are already prefixes.
+template <bool kOwn>
+__device__ __forceinline__ void scan_apply_body(const ScanArray& a, index_t block)
 {
     __shared__ index_t shared[16];
+    index_t before = 0;
+    if (kOwn)
+    {
+        index_t local = 0;
+        for (index_t k = threadIdx.x; k < block; k += kBlock) local += a.tile_sums[k];
+        before = block_sum(local, shared);
+    }
+    else
+        before = a.tile_sums[block];
     const std::int64_t base =
         static_cast<std::int64_t>(block) * kScanTile + threadIdx.x * kScanPerThread;
     index_t v[kScanPerThread];
@@ -116,25 +137,60 @@ static __device__ __forceinline__ void scan_apply_body(const index_t* input, std
 #pragma unroll
     for (int k = 0; k < kScanPerThread; ++k)
     {
-        v[k] = base + k < count ? input[base + k] : 0;
+        v[k] = base + k < a.count ? a.input[base + k] : 0;
         local += v[k];
     }
     index_t total;
-    index_t running = tile_prefix[block] + block_exclusive_sum(local, shared, &total);
+    index_t running = before + block_exclusive_sum(local, shared, &total);
 #pragma unroll
     for (int k = 0; k < kScanPerThread; ++k)
     {
-        if (base + k < count) output[base + k] = running;
+        if (base + k < a.count) a.output[base + k] = running;
         running += v[k];
     }
 }
 
-static __global__ void __launch_bounds__(kBlock) scan_apply_kernel(
-    const index_t* input, std::int64_t count, const index_t* __restrict__ tile_prefix,
-    index_t* output, const index_t* rebuild, const index_t* status)
+template <bool kOwn>
+__global__ void __launch_bounds__(kBlock) scan_apply_kernel(ScanArray first, ScanArray second,
+                                                            index_t first_tiles,
+                                                            const index_t* rebuild,
+                                                            const index_t* status)
 {
     if (!rebuilding(rebuild, status)) return;
-    scan_apply_body(input, count, tile_prefix, output, static_cast<index_t>(blockIdx.x));
+    const index_t block = static_cast<index_t>(blockIdx.x);
+    if (block < first_tiles)
+        scan_apply_body<kOwn>(first, block);
+    else
+        scan_apply_body<kOwn>(second, block - first_tiles);
+}
+
+// Exclusive scans of one array or of two (second.count 0: none); returns NDN_OK or NDN_ERR_HIP.
+inline int exclusive_scans(const ScanArray& first, const ScanArray& second,
+                           const index_t* rebuild, const index_t* status, hipStream_t stream)
+{
+    const std::int64_t tiles = scan_tiles(first.count);
+    const std::int64_t more = scan_tiles(second.count);
+    const unsigned blocks = static_cast<unsigned>(tiles + more);
+    const index_t split = static_cast<index_t>(tiles);
+    scan_tile_sums_kernel<<<blocks, kBlock, 0, stream>>>(first, second, split, rebuild, status);
+    NDN_LAUNCHED("scan_tile_sums");
+    if (std::max(tiles, more) <= kScanOwnTiles)
+    {
+        scan_apply_kernel<true><<<blocks, kBlock, 0, stream>>>(first, second, split, rebuild,
+                                                               status);
+        NDN_LAUNCHED("scan_apply");
+        return NDN_OK;
+    }
+    scan_tile_prefix_kernel<<<1, kBlock, 0, stream>>>(first.tile_sums, tiles, rebuild, status);
+    NDN_LAUNCHED("scan_tile_prefix");
+    if (more > 0)
+    {
+        scan_tile_prefix_kernel<<<1, kBlock, 0, stream>>>(second.tile_sums, more, rebuild, status);
+        NDN_LAUNCHED("scan_tile_prefix");
+    }
+    scan_apply_kernel<false><<<blocks, kBlock, 0, stream>>>(first, second, split, rebuild, status);
+    NDN_LAUNCHED("scan_apply");
+    return NDN_OK;
 }
 
 // Exclusive scan of `count` values; returns NDN_OK or NDN_ERR_HIP.
@@ -142,17 +198,9 @@ inline int exclusive_scan(const index_t* input, index_t* output, std::int64_t co
                           std::uint8_t* scan_temp, const index_t* rebuild, const index_t* status,
                           hipStream_t stream)
 {
-    const std::int64_t tiles = scan_tiles(count);
-    index_t* tile_sums = reinterpret_cast<index_t*>(scan_temp + kHeaderBytes);
-    scan_tile_sums_kernel<<<static_cast<unsigned>(tiles), kBlock, 0, stream>>>(
-        input, count, tile_sums, rebuild, status);
-    NDN_LAUNCHED("scan_tile_sums");
-    scan_tile_prefix_kernel<<<1, kBlock, 0, stream>>>(tile_sums, tiles, rebuild, status);
-    NDN_LAUNCHED("scan_tile_prefix");
-    scan_apply_kernel<<<static_cast<unsigned>(tiles), kBlock, 0, stream>>>(
-        input, count, tile_sums, output, rebuild, status);
-    NDN_LAUNCHED("scan_apply");
-    return NDN_OK;
+    const ScanArray array{input, output, count,
+                          reinterpret_cast<index_t*>(scan_temp + kHeaderBytes)};
+    return exclusive_scans(array, ScanArray{}, rebuild, status, stream);
 }
 
 }  // namespace ndn

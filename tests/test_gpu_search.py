@@ -61,3 +61,40 @@ def test_search_at_its_edges(device, dtype, npdt, kind, cell):
             both = np.concatenate([half, half[:, ::-1]])
             key = lambda a: a[np.lexsort((a[:, 1], a[:, 0]))]  # noqa: E731
             np.testing.assert_array_equal(key(got), key(both))
+
+
+@pytest.mark.parametrize("dims", [161, 162])
+def test_scan_of_many_bins(device, dims):
+    """The bins' scan with each block adding up the tile sums before it (161^3 bins, 4,076 tiles)
+    and with a launch that scans them (162^3 bins, 4,152 tiles)."""
+    cell = np.full(3, dims * 0.1 + 0.01, dtype=np.float32)
+    rng = np.random.default_rng(3)
+    x = (rng.uniform(0, 1, (4000, 3)) * cell).astype(np.float32)
+    x[::2] = x[1::2] + rng.normal(0, 0.02, (2000, 3))  # a neighbor for most atoms
+    wrapped, _ = on.wrap(x, cell)
+    ref = on.build(wrapped, cell, np.float32(0.1), capacity_multiplier=1.25)
+    nl = NeighborList(0.1)
+    nl.allocate(torch.tensor(x, device=device), torch.tensor(cell, device=device))
+    assert nl._device.buffers["bin_counts"].numel() == dims**3 + 1
+    assert ref.pair_total > 1000
+    np.testing.assert_array_equal(nl.tensors().index.cpu().numpy(), ref.pairs)
+
+
+@pytest.mark.parametrize("n", [65472, 65473, 70000])
+def test_scan_of_many_slices(device, n):
+    """The slices' scan, in the columns' launches, over one tile and over two: 1,024 entries, one
+    more, and some more. Each slice is 64 times as long as its longest row, the last the total."""
+    rng = np.random.default_rng(n)
+    cell = np.full(3, (n / 21.0) ** (1 / 3), dtype=np.float32)
+    x = (rng.uniform(0, 1, (n, 3)) * cell).astype(np.float32)
+    nl = NeighborList(0.5)
+    nl.allocate(torch.tensor(x, device=device), torch.tensor(cell, device=device))
+    wrapped, _ = on.wrap(x, cell)
+    ref = on.build(wrapped, cell, np.float32(0.5), capacity_multiplier=1.25)
+    np.testing.assert_array_equal(nl.tensors().index.cpu().numpy(), ref.pairs)
+    rows = nl.tensors().full
+    counts, slices = rows.counts.cpu().numpy(), rows.slices.cpu().numpy()
+    padded = np.zeros(-(-n // 64) * 64, np.int64)
+    padded[:n] = counts
+    np.testing.assert_array_equal(np.diff(slices), 64 * padded.reshape(-1, 64).max(axis=1))
+    assert slices[0] == 0 and counts.sum() == 2 * ref.pair_total
