@@ -234,6 +234,39 @@ int ndn_pair_parameter_vjp_frames(int dtype, const void* positions, const void* 
                                   const void* grad_virial, double* out, int64_t out_count,
                                   void* workspace, int64_t workspace_bytes, ndn_stream_t stream);
 
+/* ndn_pair_efw_full_frames and ndn_pair_parameter_vjp_frames over a choice of the stored frames:
+ * frame f of the call reads stored frame at[f] (int64, device; NULL: frame f) of the positions,
+ * cells, rows or stacks of `stored` frames; results and upstream gradients are in the order of the
+ * choice. A batch of a fit needs no copies of its frames. An entry outside [0, stored) is skipped.
+ * Workspaces as for the calls without a choice. No counterpart in the reference, which indexes
+ * its stacks (training/_fit.py:245-271). */
+int ndn_pair_efw_full_frames_at(int dtype, const void* positions, const void* cells,
+                                int64_t stored, const int64_t* at, int64_t frames,
+                                int64_t num_atoms, const int32_t* counts, const int32_t* slices,
+                                const int32_t* index, int64_t capacity, const ndn_potential* pot,
+                                void* energy, void* forces, void* virial, void* workspace,
+                                int64_t workspace_bytes, ndn_stream_t stream);
+int ndn_pair_parameter_vjp_frames_at(int dtype, const void* positions, const void* cells,
+                                     int64_t stored, const int64_t* at, int64_t frames,
+                                     int64_t num_atoms, const int32_t* stacks, int64_t capacity,
+                                     const ndn_potential* pot, const void* grad_energy,
+                                     const void* grad_forces, const void* grad_virial,
+                                     double* out, int64_t out_count, void* workspace,
+                                     int64_t workspace_bytes, ndn_stream_t stream);
+
+/* The supervised loss of F frames and its gradients (training/_loss.py:105-125): for each of the
+ * channels energy [F], forces [F, N, 3] and virial [F, 3, 3] with labels (labels[c] NULL: not in
+ * the loss; the labels are of the stored frames, read through `at` as above), term_c = sum_f
+ * coefficient mean(((predicted - label) / scale)^2) and loss = sum_c weight_c term_c. gradients[c]
+ * takes d loss / d predicted; terms [4] (T, device) the loss and the three terms. The arrays of
+ * three pointers and numbers are on the host. The workspace is ndn_frames_loss_bytes. */
+int64_t ndn_frames_loss_bytes(int64_t frames, int64_t num_atoms);
+int ndn_frames_loss(int dtype, int64_t frames, int64_t num_atoms, int64_t stored,
+                    const int64_t* at, const void* const* predicted, const void* const* labels,
+                    const double* weights, const double* scales, double coefficient,
+                    void* const* gradients, void* terms, void* workspace,
+                    int64_t workspace_bytes, ndn_stream_t stream);
+
 /* ndn_pair_efw without the workspace argument, for callers that cannot allocate device memory
  * (code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc). No
  * counterpart in the reference. Its scratch (the potential's coefficients, then 64 bytes per

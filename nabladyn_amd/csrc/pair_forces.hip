@@ -336,7 +336,8 @@ __global__ void __launch_bounds__(kSplit > 4 ? kSplit * kWave : kBlock) full_row
     const T* __restrict__ positions, const T* __restrict__ cell, const index_t* __restrict__ rows,
     const index_t* __restrict__ counts, const index_t* __restrict__ slices,
     const index_t* __restrict__ index, std::int64_t capacity, index_t num_atoms,
-    T cutoff_squared, Pot pot, T* __restrict__ forces, double* __restrict__ partials)
+    T cutoff_squared, Pot pot, FrameChoice choice, T* __restrict__ forces,
+    double* __restrict__ partials)
 {
     constexpr int kAhead = full_rows_ahead<T, Pot>();
     __shared__ double shared[16];
@@ -344,16 +345,22 @@ __global__ void __launch_bounds__(kSplit > 4 ? kSplit * kWave : kBlock) full_row
     stage_in_block(pot, staged);
     const std::int64_t slices_total = (static_cast<std::int64_t>(num_atoms) + kWave - 1) / kWave;
     // frames of one system (blockIdx.y): each frame's arrays follow the previous frame's (rows
-    // [N], counts [N], slices [N / 64 + 1], `capacity` index entries)
-    const std::int64_t frame = blockIdx.y;
+    // [N], counts [N], slices [N / 64 + 1], `capacity` index entries); the results are in the
+    // order of the choice, the frames read where it points
+    const std::int64_t frame = choice.frame(blockIdx.y);
+    partials += 8LL * blockIdx.y * gridDim.x;
+    if (frame < 0)
+    {
+        if (threadIdx.x < 8) partials[8LL * blockIdx.x + threadIdx.x] = 0.0;
+        return;
+    }
     positions += 3 * frame * num_atoms;
     cell += 3 * frame;
     if (rows != nullptr) rows += frame * num_atoms;
     counts += frame * num_atoms;
     slices += frame * (slices_total + 1);
     index += frame * capacity;
-    if (kForces) forces += 3 * frame * num_atoms;
-    partials += 8 * frame * gridDim.x;
+    if (kForces) forces += 3LL * blockIdx.y * num_atoms;
     const T lx = cell[0], ly = cell[1], lz = cell[2];
     // a distance inside every potential's domain, for the terms of entries that are not pairs
     const T safe_r2 = T(0.25) * cutoff_squared;
@@ -647,46 +654,50 @@ template <typename T, class Pot, int kSplit>
 void launch_full_split(const T* x, const T* cell, const index_t* rows, const index_t* counts,
                        const index_t* slices, const index_t* index, std::int64_t capacity,
                        index_t num_atoms, T cutoff_squared, const Pot& pot, T* forces, bool virial,
-                       double* partials, const dim3& blocks, hipStream_t stream)
+                       double* partials, const dim3& blocks, FrameChoice choice, hipStream_t stream)
 {
     constexpr int kThreads = kSplit > 4 ? kSplit * kWave : kBlock;
     const std::size_t lds = staged_bytes(pot);
     if (forces && virial)
         full_rows_kernel<T, Pot, true, true, kSplit><<<blocks, kThreads, lds, stream>>>(
             x, cell, rows, counts, slices, index, capacity, num_atoms, cutoff_squared, pot,
-            forces, partials);
+            choice, forces, partials);
     else if (forces)
         full_rows_kernel<T, Pot, true, false, kSplit><<<blocks, kThreads, lds, stream>>>(
             x, cell, rows, counts, slices, index, capacity, num_atoms, cutoff_squared, pot,
-            forces, partials);
+            choice, forces, partials);
     else if (virial)
         full_rows_kernel<T, Pot, false, true, kSplit><<<blocks, kThreads, lds, stream>>>(
             x, cell, rows, counts, slices, index, capacity, num_atoms, cutoff_squared, pot,
-            forces, partials);
+            choice, forces, partials);
     else
         full_rows_kernel<T, Pot, false, false, kSplit><<<blocks, kThreads, lds, stream>>>(
             x, cell, rows, counts, slices, index, capacity, num_atoms, cutoff_squared, pot,
-            forces, partials);
+            choice, forces, partials);
 }
 
 template <typename T, class Pot>
 void launch_full(const T* x, const T* cell, const index_t* rows, const index_t* counts,
                  const index_t* slices, const index_t* index, std::int64_t capacity,
                  index_t num_atoms, T cutoff_squared, const Pot& pot, T* forces, bool virial,
-                 double* partials, hipStream_t stream, int frames = 1)
+                 double* partials, hipStream_t stream, int frames = 1,
+                 FrameChoice choice = FrameChoice{})
 {
     const int split = full_split(num_atoms, frames);
     const dim3 blocks(static_cast<unsigned>(full_blocks(num_atoms, frames, split)),
                       static_cast<unsigned>(frames));
     if (split == 1)
         launch_full_split<T, Pot, 1>(x, cell, rows, counts, slices, index, capacity, num_atoms,
-                                     cutoff_squared, pot, forces, virial, partials, blocks, stream);
+                                     cutoff_squared, pot, forces, virial, partials, blocks, choice,
+                                     stream);
     else if (split == 4)
         launch_full_split<T, Pot, 4>(x, cell, rows, counts, slices, index, capacity, num_atoms,
-                                     cutoff_squared, pot, forces, virial, partials, blocks, stream);
+                                     cutoff_squared, pot, forces, virial, partials, blocks, choice,
+                                     stream);
     else
         launch_full_split<T, Pot, 16>(x, cell, rows, counts, slices, index, capacity, num_atoms,
-                                      cutoff_squared, pot, forces, virial, partials, blocks, stream);
+                                      cutoff_squared, pot, forces, virial, partials, blocks, choice,
+                                     stream);
 }
 
 template <typename T>
@@ -726,7 +737,8 @@ int pair_efw_full_frames_impl(const void* positions, const void* cells, std::int
                               std::int64_t num_atoms, const index_t* counts,
                               const index_t* slices, const index_t* index,
                               std::int64_t capacity, const ndn_potential* pot, void* energy,
-                              void* forces, void* virial, void* workspace, hipStream_t stream)
+                              void* forces, void* virial, void* workspace, hipStream_t stream,
+                              FrameChoice choice = FrameChoice{})
 {
     PotentialView<T> view;
     const int prepared = prepare_potential<T>(pot, workspace, stream, &view);
@@ -741,13 +753,16 @@ int pair_efw_full_frames_impl(const void* positions, const void* cells, std::int
     const int count = static_cast<int>(frames);
     if (view.kind == NDN_LJ)
         launch_full<T>(x, L, nullptr, counts, slices, index, capacity, n, view.cutoff_squared,
-                       view.lj, f, virial != nullptr, partials, stream, count);
+                       view.lj, f, virial != nullptr, partials, stream, count,
+                       choice);
     else if (stages(view))
         launch_full<T>(x, L, nullptr, counts, slices, index, capacity, n, view.cutoff_squared,
-                       staged_table(view.table), f, virial != nullptr, partials, stream, count);
+                       staged_table(view.table), f, virial != nullptr, partials, stream, count,
+                       choice);
     else
         launch_full<T>(x, L, nullptr, counts, slices, index, capacity, n, view.cutoff_squared,
-                       view.table, f, virial != nullptr, partials, stream, count);
+                       view.table, f, virial != nullptr, partials, stream, count,
+                       choice);
     NDN_LAUNCHED("full_rows_frames");
     if (energy == nullptr && virial == nullptr) return NDN_OK;
     finish_kernel<T><<<count, kBlock, 0, stream>>>(partials, blocks, static_cast<T*>(energy),
@@ -911,28 +926,42 @@ int ndn_pair_frames_workspace_bytes(int dtype, const ndn_potential* pot, int64_t
     return NDN_OK;
 }
 
-int ndn_pair_efw_full_frames(int dtype, const void* positions, const void* cells, int64_t frames,
-                             int64_t num_atoms, const int32_t* counts, const int32_t* slices,
-                             const int32_t* index, int64_t capacity, const ndn_potential* pot,
-                             void* energy, void* forces, void* virial, void* workspace,
-                             int64_t workspace_bytes, ndn_stream_t stream)
+int ndn_pair_efw_full_frames_at(int dtype, const void* positions, const void* cells,
+                                int64_t stored, const int64_t* at, int64_t frames,
+                                int64_t num_atoms, const int32_t* counts, const int32_t* slices,
+                                const int32_t* index, int64_t capacity, const ndn_potential* pot,
+                                void* energy, void* forces, void* virial, void* workspace,
+                                int64_t workspace_bytes, ndn_stream_t stream)
 {
     const int checked = check_potential(pot, num_atoms);
     if (checked != NDN_OK) return checked;
     NDN_REQUIRE(positions && cells && counts && slices && index && workspace, "a buffer is null");
     NDN_REQUIRE(num_atoms >= 1 && num_atoms <= INT32_MAX, "N must satisfy 1 <= N < 2**31");
     NDN_REQUIRE(capacity >= 1, "each frame's full list must have a positive capacity");
+    NDN_REQUIRE(at == nullptr || stored >= 1, "a choice of frames needs stored frames");
     std::int64_t needed = 0;
     const int sized = ndn_pair_frames_workspace_bytes(dtype, pot, frames, num_atoms, &needed);
     if (sized != NDN_OK) return sized;
     NDN_REQUIRE(workspace_bytes >= needed, "the workspace is too small");
+    const FrameChoice choice{at, stored};
     if (dtype == NDN_F32)
         return pair_efw_full_frames_impl<float>(positions, cells, frames, num_atoms, counts, slices,
                                                 index, capacity, pot, energy, forces, virial,
-                                                workspace, stream);
+                                                workspace, stream, choice);
     return pair_efw_full_frames_impl<double>(positions, cells, frames, num_atoms, counts, slices,
                                              index, capacity, pot, energy, forces, virial,
-                                             workspace, stream);
+                                             workspace, stream, choice);
+}
+
+int ndn_pair_efw_full_frames(int dtype, const void* positions, const void* cells, int64_t frames,
+                             int64_t num_atoms, const int32_t* counts, const int32_t* slices,
+                             const int32_t* index, int64_t capacity, const ndn_potential* pot,
+                             void* energy, void* forces, void* virial, void* workspace,
+                             int64_t workspace_bytes, ndn_stream_t stream)
+{
+    return ndn_pair_efw_full_frames_at(dtype, positions, cells, frames, nullptr, frames, num_atoms,
+                                       counts, slices, index, capacity, pot, energy, forces,
+                                       virial, workspace, workspace_bytes, stream);
 }
 
 int ndn_pair_efw_frames(int dtype, const void* positions, const void* cells, int64_t frames,

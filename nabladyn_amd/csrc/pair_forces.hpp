@@ -34,6 +34,22 @@ __device__ __forceinline__ T exact_squared(T dx, T dy, T dz)
     return (xx + yy) + zz;
 }
 
+// Which of the stored frames a launch over frames reads: frame f of the launch is stored frame
+// at[f], or f itself without a choice. An entry outside the stored frames gives -1, and its block
+// does nothing.
+struct FrameChoice
+{
+    const std::int64_t* at = nullptr;
+    std::int64_t stored = 0;
+
+    __device__ __forceinline__ std::int64_t frame(unsigned f) const
+    {
+        if (at == nullptr) return f;
+        const std::int64_t chosen = at[f];
+        return chosen >= 0 && chosen < stored ? chosen : -1;
+    }
+};
+
 template <typename T>
 struct PotentialView
 {

@@ -226,16 +226,18 @@ __global__ void __launch_bounds__(kBlock) lj_parameter_kernel(
     const T* __restrict__ positions, const T* __restrict__ cell, const index_t* __restrict__ pairs,
     std::int64_t capacity, index_t num_atoms, T cutoff_squared, const T* __restrict__ sigma,
     const T* __restrict__ epsilon, const std::int64_t* __restrict__ types, int num_types,
-    const T* __restrict__ strain_matrix, Upstream<T> frames_up, double* __restrict__ out)
+    const T* __restrict__ strain_matrix, Upstream<T> frames_up, FrameChoice choice,
+    double* __restrict__ out)
 {
     __shared__ double local_store[kLocalGradient];
     const Strain<T> strain = read_strain(strain_matrix);
     // frames of one system (blockIdx.y) add into the same out
-    const std::int64_t frame = blockIdx.y;
+    const std::int64_t frame = choice.frame(blockIdx.y);
+    if (frame < 0) return;
     positions += 3 * frame * num_atoms;
     cell += 3 * frame;
     pairs += 2 * frame * capacity;
-    const Upstream<T> up = frames_up.at(frame, num_atoms);
+    const Upstream<T> up = frames_up.at(blockIdx.y, num_atoms);
     const int rows = num_types * (num_types + 1) / 2;
     double* local = 2 * rows <= kLocalGradient ? local_store : nullptr;
     if (local != nullptr)
@@ -286,15 +288,17 @@ template <typename T, bool kStrained>
 __global__ void __launch_bounds__(kBlock) table_parameter_kernel(
     const T* __restrict__ positions, const T* __restrict__ cell, const index_t* __restrict__ pairs,
     std::int64_t capacity, index_t num_atoms, T cutoff_squared, Table<T> table,
-    const T* __restrict__ strain_matrix, Upstream<T> frames_up, double* __restrict__ out)
+    const T* __restrict__ strain_matrix, Upstream<T> frames_up, FrameChoice choice,
+    double* __restrict__ out)
 {
     __shared__ double local_store[kLocalGradient];
     const Strain<T> strain = read_strain(strain_matrix);
-    const std::int64_t frame = blockIdx.y;
+    const std::int64_t frame = choice.frame(blockIdx.y);
+    if (frame < 0) return;
     positions += 3 * frame * num_atoms;
     cell += 3 * frame;
     pairs += 2 * frame * capacity;
-    const Upstream<T> up = frames_up.at(frame, num_atoms);
+    const Upstream<T> up = frames_up.at(blockIdx.y, num_atoms);
     const int knots = table.knots;
     const int rows = table.num_types * (table.num_types + 1) / 2;
     const std::int64_t entries = static_cast<std::int64_t>(rows) * knots;
@@ -434,7 +438,7 @@ int parameter_impl(const void* positions, const void* cell, std::int64_t num_ato
                    const index_t* pairs, std::int64_t capacity, const ndn_potential* pot,
                    const void* strain, const Upstream<T>& up, double* out,
                    std::int64_t out_count, void* workspace, hipStream_t stream,
-                   std::int64_t frames = 1)
+                   std::int64_t frames = 1, FrameChoice choice = FrameChoice{})
 {
     PotentialView<T> view;
     const int prepared = prepare_potential<T>(pot, workspace, stream, &view);
@@ -459,18 +463,18 @@ int parameter_impl(const void* positions, const void* cell, std::int64_t num_ato
         if (strained)
             lj_parameter_kernel<T, true><<<blocks, kBlock, 0, stream>>>(
                 x, L, pairs, capacity, n, view.cutoff_squared, sigma, epsilon, pot->atom_types,
-                pot->num_types, e, up, out);
+                pot->num_types, e, up, choice, out);
         else
             lj_parameter_kernel<T, false><<<blocks, kBlock, 0, stream>>>(
                 x, L, pairs, capacity, n, view.cutoff_squared, sigma, epsilon, pot->atom_types,
-                pot->num_types, e, up, out);
+                pot->num_types, e, up, choice, out);
     }
     else if (strained)
         table_parameter_kernel<T, true><<<blocks, kBlock, 0, stream>>>(
-            x, L, pairs, capacity, n, view.cutoff_squared, view.table, e, up, out);
+            x, L, pairs, capacity, n, view.cutoff_squared, view.table, e, up, choice, out);
     else
         table_parameter_kernel<T, false><<<blocks, kBlock, 0, stream>>>(
-            x, L, pairs, capacity, n, view.cutoff_squared, view.table, e, up, out);
+            x, L, pairs, capacity, n, view.cutoff_squared, view.table, e, up, choice, out);
     NDN_LAUNCHED("parameter_gradient");
     return NDN_OK;
 }
@@ -497,7 +501,7 @@ int vjp_call(int dtype, const void* positions, const void* cells, std::int64_t f
              std::int64_t num_atoms, const int32_t* pairs, std::int64_t capacity,
              const ndn_potential* pot, const void* grad_energy, const void* grad_forces,
              const void* grad_virial, double* out, std::int64_t out_count, void* workspace,
-             hipStream_t stream)
+             hipStream_t stream, FrameChoice choice = FrameChoice{})
 {
     const std::int64_t rows = static_cast<std::int64_t>(pot->num_types) * (pot->num_types + 1) / 2;
     const std::int64_t expected = pot->kind == NDN_LJ ? 2 * rows : rows * pot->knots;
@@ -509,13 +513,118 @@ int vjp_call(int dtype, const void* positions, const void* cells, std::int64_t f
             Upstream<float>{static_cast<const float*>(grad_energy),
                             static_cast<const float*>(grad_forces),
                             static_cast<const float*>(grad_virial), false},
-            out, out_count, workspace, stream, frames);
+            out, out_count, workspace, stream, frames, choice);
     return parameter_impl<double>(
         positions, cells, num_atoms, pairs, capacity, pot, nullptr,
         Upstream<double>{static_cast<const double*>(grad_energy),
                          static_cast<const double*>(grad_forces),
                          static_cast<const double*>(grad_virial), false},
-        out, out_count, workspace, stream, frames);
+        out, out_count, workspace, stream, frames, choice);
+}
+
+// ---- the supervised loss over frames ---------------------------------------------------------
+
+// The energy, force and virial channels of a launch (labels null: not in the loss).
+template <typename T>
+struct LossChannels
+{
+    const T* predicted[3];
+    const T* labels[3];    // of the stored frames
+    T* gradients[3];       // d loss / d predicted
+    T scale[3];            // the squares are of (predicted - label) / scale
+    T factor[3];           // 2 weight coefficient / (scale^2 components)
+    std::int64_t components[3];  // per frame: 1, 3N, 9
+};
+
+// Blocks per frame: a block for each 4,096 of its force components, at most 64.
+std::int64_t loss_blocks(std::int64_t num_atoms)
+{
+    return std::max<std::int64_t>(1, std::min<std::int64_t>((3 * num_atoms + 4095) / 4096, 64));
+}
+
+// Each channel's gradient, and the block's sums of squares (fp64, a fixed order) into its slot:
+// what autograd does in some forty small launches an update, each its own pass over the forces.
+template <typename T>
+__global__ void __launch_bounds__(kBlock) frames_loss_kernel(LossChannels<T> c, FrameChoice choice,
+                                                             double* __restrict__ partials)
+{
+    __shared__ double shared[16];
+    const std::int64_t frame = choice.frame(blockIdx.y);
+    double* out = partials + 3 * (static_cast<std::int64_t>(blockIdx.y) * gridDim.x + blockIdx.x);
+    for (int k = 0; k < 3; ++k)
+    {
+        double sum = 0.0;
+        if (c.labels[k] != nullptr && frame >= 0)
+        {
+            const std::int64_t n = c.components[k];
+            const T* predicted = c.predicted[k] + blockIdx.y * n;
+            const T* labels = c.labels[k] + frame * n;
+            T* gradients = c.gradients[k] + blockIdx.y * n;
+            const std::int64_t stride = static_cast<std::int64_t>(gridDim.x) * kBlock;
+            for (std::int64_t i = static_cast<std::int64_t>(blockIdx.x) * kBlock + threadIdx.x;
+                 i < n; i += stride)
+            {
+                const T error = predicted[i] - labels[i];
+                const T scaled = error / c.scale[k];
+                sum += static_cast<double>(scaled) * static_cast<double>(scaled);
+                gradients[i] = c.factor[k] * error;
+            }
+        }
+        sum = block_sum(sum, shared);
+        if (threadIdx.x == 0) out[k] = sum;
+    }
+}
+
+// terms [4]: the loss and the three unweighted terms, sum_f coefficient mean_f.
+template <typename T>
+__global__ void __launch_bounds__(kBlock) frames_loss_finish_kernel(
+    const double* __restrict__ partials, std::int64_t slots, double share_e, double share_f,
+    double share_w, double weight_e, double weight_f, double weight_w, T* __restrict__ terms)
+{
+    __shared__ double shared[16];
+    double sums[3] = {0, 0, 0};
+    for (std::int64_t s = threadIdx.x; s < slots; s += kBlock)
+        for (int k = 0; k < 3; ++k) sums[k] += partials[3 * s + k];
+    for (int k = 0; k < 3; ++k) sums[k] = block_sum(sums[k], shared);
+    if (threadIdx.x != 0) return;
+    const double e = share_e * sums[0], f = share_f * sums[1], w = share_w * sums[2];
+    terms[0] = static_cast<T>((weight_e * e + weight_f * f) + weight_w * w);
+    terms[1] = static_cast<T>(e);
+    terms[2] = static_cast<T>(f);
+    terms[3] = static_cast<T>(w);
+}
+
+template <typename T>
+int loss_impl(std::int64_t frames, std::int64_t num_atoms, FrameChoice choice,
+              const void* const* predicted, const void* const* labels, const double* weights,
+              const double* scales, double coefficient, void* const* gradients, void* terms,
+              void* workspace, hipStream_t stream)
+{
+    LossChannels<T> c{};
+    double share[3] = {0, 0, 0}, weight[3] = {0, 0, 0};
+    const std::int64_t components[3] = {1, 3 * num_atoms, 9};
+    for (int k = 0; k < 3; ++k)
+    {
+        c.components[k] = components[k];
+        c.labels[k] = static_cast<const T*>(labels[k]);
+        if (labels[k] == nullptr) continue;
+        c.predicted[k] = static_cast<const T*>(predicted[k]);
+        c.gradients[k] = static_cast<T*>(gradients[k]);
+        c.scale[k] = static_cast<T>(scales[k]);
+        share[k] = coefficient / static_cast<double>(components[k]);
+        weight[k] = weights[k];
+        c.factor[k] = static_cast<T>(2.0 * weights[k] * share[k] / (scales[k] * scales[k]));
+    }
+    auto* partials = static_cast<double*>(workspace);
+    const std::int64_t blocks = loss_blocks(num_atoms);
+    frames_loss_kernel<T><<<dim3(static_cast<unsigned>(blocks), static_cast<unsigned>(frames)),
+                            kBlock, 0, stream>>>(c, choice, partials);
+    NDN_LAUNCHED("frames_loss");
+    frames_loss_finish_kernel<T><<<1, kBlock, 0, stream>>>(
+        partials, blocks * frames, share[0], share[1], share[2], weight[0], weight[1], weight[2],
+        static_cast<T*>(terms));
+    NDN_LAUNCHED("frames_loss_finish");
+    return NDN_OK;
 }
 
 }  // namespace ndn
@@ -575,6 +684,24 @@ int ndn_pair_parameter_vjp(int dtype, const void* positions, const void* cell, i
                     grad_forces, grad_virial, out, out_count, workspace, stream);
 }
 
+int ndn_pair_parameter_vjp_frames_at(int dtype, const void* positions, const void* cells,
+                                     int64_t stored, const int64_t* at, int64_t frames,
+                                     int64_t num_atoms, const int32_t* stacks, int64_t capacity,
+                                     const ndn_potential* pot, const void* grad_energy,
+                                     const void* grad_forces, const void* grad_virial,
+                                     double* out, int64_t out_count, void* workspace,
+                                     int64_t workspace_bytes, ndn_stream_t stream)
+{
+    const int checked = check_pair_call(dtype, pot, positions, cells, num_atoms, stacks, capacity,
+                                        workspace, workspace_bytes);
+    if (checked != NDN_OK) return checked;
+    NDN_REQUIRE(frames >= 1 && frames <= 65535, "frames must lie in [1, 65535]");
+    NDN_REQUIRE(at == nullptr || stored >= 1, "a choice of frames needs stored frames");
+    return vjp_call(dtype, positions, cells, frames, num_atoms, stacks, capacity, pot,
+                    grad_energy, grad_forces, grad_virial, out, out_count, workspace, stream,
+                    FrameChoice{at, stored});
+}
+
 int ndn_pair_parameter_vjp_frames(int dtype, const void* positions, const void* cells,
                                   int64_t frames, int64_t num_atoms, const int32_t* stacks,
                                   int64_t capacity, const ndn_potential* pot,
@@ -582,12 +709,40 @@ int ndn_pair_parameter_vjp_frames(int dtype, const void* positions, const void* 
                                   const void* grad_virial, double* out, int64_t out_count,
                                   void* workspace, int64_t workspace_bytes, ndn_stream_t stream)
 {
-    const int checked = check_pair_call(dtype, pot, positions, cells, num_atoms, stacks, capacity,
-                                        workspace, workspace_bytes);
-    if (checked != NDN_OK) return checked;
+    return ndn_pair_parameter_vjp_frames_at(dtype, positions, cells, frames, nullptr, frames,
+                                            num_atoms, stacks, capacity, pot, grad_energy,
+                                            grad_forces, grad_virial, out, out_count, workspace,
+                                            workspace_bytes, stream);
+}
+
+int64_t ndn_frames_loss_bytes(int64_t frames, int64_t num_atoms)
+{
+    return frames * loss_blocks(num_atoms) * 3 * static_cast<int64_t>(sizeof(double));
+}
+
+int ndn_frames_loss(int dtype, int64_t frames, int64_t num_atoms, int64_t stored,
+                    const int64_t* at, const void* const* predicted, const void* const* labels,
+                    const double* weights, const double* scales, double coefficient,
+                    void* const* gradients, void* terms, void* workspace,
+                    int64_t workspace_bytes, ndn_stream_t stream)
+{
+    NDN_REQUIRE(predicted && labels && weights && scales && gradients && terms && workspace,
+                "a buffer is null");
     NDN_REQUIRE(frames >= 1 && frames <= 65535, "frames must lie in [1, 65535]");
-    return vjp_call(dtype, positions, cells, frames, num_atoms, stacks, capacity, pot,
-                    grad_energy, grad_forces, grad_virial, out, out_count, workspace, stream);
+    NDN_REQUIRE(num_atoms >= 1 && num_atoms <= INT32_MAX, "N must satisfy 1 <= N < 2**31");
+    NDN_REQUIRE(at == nullptr || stored >= 1, "a choice of frames needs stored frames");
+    NDN_REQUIRE(workspace_bytes >= ndn_frames_loss_bytes(frames, num_atoms),
+                "the workspace is too small");
+    for (int c = 0; c < 3; ++c)
+        NDN_REQUIRE(labels[c] == nullptr || (predicted[c] && gradients[c] && scales[c] != 0.0),
+                    "a labeled channel needs its prediction, gradient and a nonzero scale");
+    const FrameChoice choice{at, stored};
+    if (dtype == NDN_F32)
+        return loss_impl<float>(frames, num_atoms, choice, predicted, labels, weights, scales,
+                                coefficient, gradients, terms, workspace, stream);
+    NDN_REQUIRE(dtype == NDN_F64, "dtype must be NDN_F32 or NDN_F64");
+    return loss_impl<double>(frames, num_atoms, choice, predicted, labels, weights, scales,
+                             coefficient, gradients, terms, workspace, stream);
 }
 
 }  // extern "C"

@@ -154,21 +154,25 @@ def evaluate_frames(model, positions: Tensor, cells: Tensor, stacks: Tensor, nat
     return e, f, w
 
 
-def evaluate_frames_full(model, positions: Tensor, cells: Tensor, rows, native):
+def evaluate_frames_full(model, positions: Tensor, cells: Tensor, rows, native,
+                         at: Tensor | None = None):
     """``evaluate_frames`` over full rows (``rows``: counts [F, N], slices [F, N / 64 + 1] and
     index [F, capacity], int32, the layout ``training._loss.frame_rows`` builds): a lane per
-    row, no atomics."""
+    row, no atomics. With ``at`` (int64 [B], on the device) the results are those of the stored
+    frames it names, which are read in place."""
     x = positions.detach().contiguous()
     cells = cells.detach().contiguous()
-    frames, atoms = x.shape[0], x.shape[1]
+    stored, atoms = x.shape[0], x.shape[1]
+    frames = stored if at is None else at.numel()
     dtype, device = x.dtype, x.device
     workspace, pot, keep = _frames_workspace(model, frames, atoms, device, native)
     e = torch.empty(frames, dtype=dtype, device=device)
     f = torch.empty((frames, atoms, 3), dtype=dtype, device=device)
     w = torch.empty((frames, 3, 3), dtype=dtype, device=device)
     counts, slices, index = rows
-    _native.call("pair_efw_full_frames", _native.dtype_tag(dtype), _native.ptr(x),
-                 _native.ptr(cells), _native.ctypes.c_int64(frames), _native.ctypes.c_int64(atoms),
+    _native.call("pair_efw_full_frames_at", _native.dtype_tag(dtype), _native.ptr(x),
+                 _native.ptr(cells), _native.ctypes.c_int64(stored), _native.ptr(at),
+                 _native.ctypes.c_int64(frames), _native.ctypes.c_int64(atoms),
                  _native.ptr(counts), _native.ptr(slices), _native.ptr(index),
                  _native.ctypes.c_int64(index.shape[1]), _native.ctypes.byref(pot), _native.ptr(e),
                  _native.ptr(f), _native.ptr(w), _native.ptr(workspace),
@@ -178,12 +182,14 @@ def evaluate_frames_full(model, positions: Tensor, cells: Tensor, rows, native):
 
 
 def parameter_vjp_frames(model, positions: Tensor, cells: Tensor, stacks: Tensor, grad_energy,
-                         grad_forces, grad_virial, native) -> Tensor:
-    """``parameter_vjp`` summed over the frames of ``evaluate_frames``; upstream gradients
-    [F], [F, N, 3], [F, 3, 3], each may be None."""
+                         grad_forces, grad_virial, native, at: Tensor | None = None) -> Tensor:
+    """``parameter_vjp`` summed over the frames of ``evaluate_frames``, or over those that ``at``
+    names (as for ``evaluate_frames_full``); upstream gradients [F], [F, N, 3], [F, 3, 3], each
+    may be None."""
     x = positions.detach().contiguous()
     cells = cells.detach().contiguous()
-    frames, atoms = x.shape[0], x.shape[1]
+    stored, atoms = x.shape[0], x.shape[1]
+    frames = stored if at is None else at.numel()
     workspace, pot, keep = _frames_workspace(model, frames, stacks.shape[2], x.device, native)
     out = torch.empty(model._parameter_gradient_shape(), dtype=torch.float64, device=x.device)
 
@@ -191,14 +197,45 @@ def parameter_vjp_frames(model, positions: Tensor, cells: Tensor, stacks: Tensor
         return None if g is None else g.detach().to(x.dtype).contiguous()
 
     ge, gf, gw = upstream(grad_energy), upstream(grad_forces), upstream(grad_virial)
-    _native.call("pair_parameter_vjp_frames", _native.dtype_tag(x.dtype), _native.ptr(x),
-                 _native.ptr(cells), _native.ctypes.c_int64(frames), _native.ctypes.c_int64(atoms),
+    _native.call("pair_parameter_vjp_frames_at", _native.dtype_tag(x.dtype), _native.ptr(x),
+                 _native.ptr(cells), _native.ctypes.c_int64(stored), _native.ptr(at),
+                 _native.ctypes.c_int64(frames), _native.ctypes.c_int64(atoms),
                  _native.ptr(stacks), _native.ctypes.c_int64(stacks.shape[2]),
                  _native.ctypes.byref(pot), _native.ptr(ge), _native.ptr(gf), _native.ptr(gw),
                  _native.ptr(out), _native.ctypes.c_int64(out.numel()), _native.ptr(workspace),
                  _native.ctypes.c_int64(workspace.numel()), _native.stream(x.device))
     del keep
     return out
+
+
+def frames_loss(predicted, labels, at: Tensor, weights, scales, coefficient: float):
+    """The supervised loss of B frames and its gradients, from two launches (``ndn_frames_loss``).
+
+    ``predicted`` and ``labels`` are (energy, forces, virial) triples: [B] .. of the frames that
+    ``at`` (int64 [B]) names, and of every stored frame, a label None for a channel outside the
+    loss; ``weights`` and ``scales`` are numbers, one per channel. Returns the gradients (None
+    outside the loss) and [4]: the loss and the three unweighted terms."""
+    energy, forces, _ = predicted
+    frames, atoms, device = forces.shape[0], forces.shape[1], forces.device
+    stored = next(v.shape[0] for v in labels if v is not None)
+    gradients = tuple(None if label is None else torch.empty_like(value)
+                      for value, label in zip(predicted, labels))
+    terms = torch.empty(4, dtype=forces.dtype, device=device)
+    size = _native.lib().ndn_frames_loss_bytes
+    size.restype = _native.ctypes.c_int64
+    workspace = torch.empty(size(_native.ctypes.c_int64(frames), _native.ctypes.c_int64(atoms)),
+                            dtype=torch.uint8, device=device)
+    pointers = _native.ctypes.c_void_p * 3
+    numbers = _native.ctypes.c_double * 3
+    _native.call("frames_loss", _native.dtype_tag(forces.dtype), _native.ctypes.c_int64(frames),
+                 _native.ctypes.c_int64(atoms), _native.ctypes.c_int64(stored), _native.ptr(at),
+                 pointers(*(_native.ptr(v) for v in predicted)),
+                 pointers(*(_native.ptr(v) for v in labels)), numbers(*weights), numbers(*scales),
+                 _native.ctypes.c_double(coefficient),
+                 pointers(*(_native.ptr(v) for v in gradients)), _native.ptr(terms),
+                 _native.ptr(workspace), _native.ctypes.c_int64(workspace.numel()),
+                 _native.stream(device))
+    return gradients, terms
 
 
 class _FirstOrderOnly(torch.autograd.Function):

@@ -17,7 +17,8 @@ from torch import Tensor
 
 from .. import _native, space
 from ..neighbors import NeighborList
-from ..potential import Potential
+from ..potential import LennardJones, Potential, Sum, Tabulated
+from ..potential._energy import evaluate_frames_full, frames_loss, parameter_vjp_frames
 from . import _loss
 from ._dataset import Dataset
 
@@ -173,6 +174,59 @@ def _chunks(frames: Tensor, size: int):
     yield from frames.split(size)
 
 
+def _pair_parts(model: Potential, prefix: str = ""):
+    """(parameter prefix, model) of each LJ or table in a model that is one or a sum of them,
+    None for any other (a subclass may compute otherwise)."""
+    if type(model) in (LennardJones, Tabulated):
+        return [(prefix, model)]
+    if type(model) is not Sum:
+        return None
+    parts = [_pair_parts(part, f"{prefix}parts.{k}.") for k, part in enumerate(model.parts)]
+    return None if any(part is None for part in parts) else [p for part in parts for p in part]
+
+
+def _kernel_parts(model: Potential, trained: dict[str, Tensor], prepared: _Prepared):
+    """``_pair_parts`` when the kernels alone can form the batch gradient: the trained tensors are
+    the model's own parameters and the frames have full rows; else None."""
+    own = dict(model.named_parameters())
+    if prepared.rows is None or any(own.get(name) is not value for name, value in trained.items()):
+        return None
+    return _pair_parts(model)
+
+
+def _kernel_gradient(model: Potential, parts, trained: dict[str, Tensor], prepared: _Prepared,
+                     chunk: Tensor, coefficient: float, weights: dict[str, float],
+                     channel_scales: dict[str, float]):
+    """(gradient by name, loss, terms by name) of a chunk of frames from the library's kernels
+    alone: the parts' channels, the loss with its gradients, the parts' parameter VJPs. The
+    frames, rows, stacks and labels are read in place."""
+    cutoffs = model._list_cutoffs
+    rows, stacks = dict(zip(cutoffs, prepared.rows)), dict(zip(cutoffs, prepared.stacks))
+    natives = [part._native() for _, part in parts]
+    values = None
+    for (_, part), native in zip(parts, natives):
+        found = evaluate_frames_full(part, prepared.positions, prepared.cells,
+                                     _loss._list_for(rows, part.cutoff), native, chunk)
+        values = found if values is None else tuple(a + b for a, b in zip(values, found))
+    labels = tuple(prepared.labels.get(name) for name in _loss.CHANNELS)
+    gradients, terms = frames_loss(values, labels, chunk,
+                                   [weights.get(name, 0.0) for name in _loss.CHANNELS],
+                                   [channel_scales.get(name, 1.0) for name in _loss.CHANNELS],
+                                   coefficient)
+    gradient = {}
+    for (prefix, part), native in zip(parts, natives):
+        names = [name for name, _ in part.named_parameters() if prefix + name in trained]
+        if not names:
+            continue
+        g = parameter_vjp_frames(part, prepared.positions, prepared.cells,
+                                 _loss._list_for(stacks, part.cutoff), *gradients, native, chunk)
+        split = part._split_parameter_gradient(g.to(model.dtype))
+        own = [name for name, _ in part.named_parameters()]
+        gradient.update((prefix + name, split[own.index(name)]) for name in names)
+    return gradient, terms[0], {name: terms[1 + k] for k, name in enumerate(_loss.CHANNELS)
+                                if name in prepared.labels}
+
+
 def batch_gradient(model: Potential, trained: dict[str, Tensor], prepared: _Prepared,
                    frames: Tensor, size: int, weights: dict[str, float],
                    channel_scales: dict[str, float]):
@@ -184,8 +238,20 @@ def batch_gradient(model: Potential, trained: dict[str, Tensor], prepared: _Prep
     device = prepared.positions.device
     gradient = {name: torch.zeros_like(value) for name, value in trained.items()}
     total_loss, total_terms = None, None
+    parts = _kernel_parts(model, trained, prepared)
     for chunk in _chunks(frames, size):
         chunk = chunk.to(device)
+        if parts is not None:
+            found, value, terms = _kernel_gradient(model, parts, trained, prepared, chunk,
+                                                   1.0 / len(frames), weights, channel_scales)
+            for name, g in found.items():
+                gradient[name] += g
+            if total_loss is None:
+                total_loss, total_terms = value, terms
+            else:
+                total_loss = total_loss + value
+                total_terms = {k: total_terms[k] + v for k, v in terms.items()}
+            continue
         coefficients = torch.full((len(chunk),), 1.0 / len(frames), dtype=model.dtype,
                                   device=device)
         stacks, rows = prepared.chunk(chunk)

@@ -1,0 +1,77 @@
+"""The batch gradient of a fit from the kernels alone (channels, loss and VJP over a choice of the
+stored frames) against the same through autograd, which a fit takes for parameters that are not
+the model's own: a permuted, a repeated and a partial choice of frames, each subset of the
+channels, one type, two types and a sum, force components on both sides of a loss block (1,365 and
+1,366 atoms).
+
+Tolerance. Both routes evaluate the same channels in the model's dtype and add the parameters'
+pair sums in fp64; they differ by the rounding of the upstream gradients, some 3 ulp each and
+independent over the components. fp64 1e-11 of max |g|, fp32 1e-5; the loss and its terms, sums of
+squares in another order, 1e-12 and 1e-5 of themselves."""
+
+import numpy as np
+import pytest
+import torch
+
+from nabladyn_amd import potential, training, workloads
+from nabladyn_amd.training import _fit
+
+pytestmark = pytest.mark.gpu
+
+
+def _model(kind, n, dtype, device):
+    as_t = lambda v: torch.tensor(v, dtype=dtype, device=device)  # noqa: E731
+    zeros = torch.zeros(n, dtype=torch.int64, device=device)
+    table = lambda: potential.tabulated(  # noqa: E731
+        atom_types=zeros, table=as_t(workloads.lj_table(40, noise=0.0, sigma=0.45)[None]),
+        start=as_t([0.3]), cutoff=1.2, trainable=("table",))
+    if kind == "table":
+        return table()
+    if kind == "mixture":
+        types = torch.arange(n, device=device) % 2
+        return potential.lennard_jones(atom_types=types, sigma=as_t([0.47, 0.46, 0.45]),
+                                       epsilon=as_t([3.0, 3.1, 3.2]), cutoff=1.2,
+                                       trainable=("sigma", "epsilon"))
+    lj = potential.lennard_jones(atom_types=zeros, sigma=as_t([0.46]), epsilon=as_t([2.0]),
+                                 cutoff=1.0, trainable=("epsilon",))
+    return potential.sum(lj, table())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("kind,n,channels", [
+    ("table", 1365, ("energy", "forces", "virial")), ("table", 1366, ("forces",)),
+    ("mixture", 500, ("energy", "virial")), ("mixture", 500, ("forces", "virial")),
+    ("sum", 500, ("energy", "forces", "virial")),
+])
+def test_kernel_gradient_equals_autograd(device, dtype, kind, n, channels):
+    rng = np.random.default_rng(n)
+    frames, length = 6, (n / 8.0) ** (1 / 3)
+    per = int(np.ceil(n ** (1 / 3)))
+    x = np.stack([workloads.lattice((per,) * 3, (length,) * 3, 0.04, rng, n=n)
+                  for _ in range(frames)])
+    labels = {"energy": rng.normal(0, 50, frames), "forces": rng.normal(0, 30, (frames, n, 3)),
+              "virial": rng.normal(0, 80, (frames, 3, 3))}
+    as_np = lambda v: np.asarray(v).astype(np.float32 if dtype == torch.float32 else np.float64)  # noqa: E731
+    data = training.Dataset(as_np(x), as_np(np.full((frames, 3), length)),
+                            **{k: as_np(labels[k]) for k in channels})
+    model = _model(kind, n, dtype, device)
+    prepared = _fit._prepare(model, data, channels)
+    scales = training.scales(**prepared.labels)
+    weights = {name: 0.5 + k for k, name in enumerate(channels)}
+    own = {name: p for name, p in model.named_parameters() if p.requires_grad}
+    copies = {name: p.detach().clone() for name, p in own.items()}
+    assert _fit._kernel_parts(model, own, prepared) is not None
+    assert _fit._kernel_parts(model, copies, prepared) is None
+    loose, tight = (1e-5, 1e-5) if dtype == torch.float32 else (1e-11, 1e-12)
+    for chosen, size in (([3, 0, 5, 1, 4, 2], 6), ([2, 2, 0], 3), ([4, 1, 3], 2), ([5], 1)):
+        chosen = torch.tensor(chosen)
+        g, loss, terms = _fit.batch_gradient(model, own, prepared, chosen, size, weights, scales)
+        g0, loss0, terms0 = _fit.batch_gradient(model, copies, prepared, chosen, size, weights,
+                                                scales)
+        assert set(g) == set(g0) and set(terms) == set(terms0) == set(channels)
+        for name in g:
+            assert g[name].dtype == g0[name].dtype and g[name].shape == g0[name].shape
+            assert float((g[name] - g0[name]).abs().max()) <= loose * float(g0[name].abs().max())
+        assert abs(float(loss) - float(loss0)) <= tight * abs(float(loss0))
+        for name in terms:
+            assert abs(float(terms[name]) - float(terms0[name])) <= tight * abs(float(terms0[name]))
