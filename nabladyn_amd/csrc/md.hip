@@ -252,9 +252,10 @@ struct TypedTable
 //          the tangent's slope, as the reference's);
 //   energy (0.5 a, 0.5 b, 0.5 c, 0): u = u1 + s (0.5 a + s (0.5 b + s 0.5 c)) + 0.5 a min(t, 0).
 // A pair of a kick step (no energy) reads one aligned 16-byte (fp64: 32-byte) entry. r and the
-// knot coordinate x = (r - start) / h come from the reference's own operations, each correctly
-// rounded (square root, subtraction, division), so every pair's segment and t carry the
-// reference's bits; 1/r, which only scales the force, is the hardware reciprocal.
+// knot coordinate x = (r - start) / h are the reference's: its square root, subtraction and
+// division, each correctly rounded (pair_distance; the quotient is a product corrected by its
+// remainder, which the library's root and division reach in twice the instructions); 1/r, which
+// only scales the force, is the hardware reciprocal.
 template <typename T>
 struct OneTypeTable
 {
@@ -306,13 +307,16 @@ struct OneTypeTable
     struct Bound
     {
         const V4* segments;
-        T start, h;
+        T start, h, inverse_h;
         T last;  // the last segment, K - 2
 
         __device__ __forceinline__ void eval(T, T, T r2, T& u, T& fs) const
         {
-            const T r = sqrt(r2);
-            const T x = (r - start) / h;
+            const T r = pair_distance(r2);
+            // (r - start) / h: the product with 1 / h corrected by its remainder
+            const T offset = r - start;
+            const T q = offset * inverse_h;
+            const T x = fma(fma(-q, h, offset), inverse_h, q);
             // the segment, in range whatever r2 was: the clamps send a NaN to 0, so the
             // conversion always sees a value in [0, last]
             T clamped = x > T(0) ? x : T(0);
@@ -329,7 +333,7 @@ struct OneTypeTable
 
     __device__ __forceinline__ Bound bind(const unsigned char* lds) const
     {
-        return Bound{reinterpret_cast<const V4*>(lds), start[0], spacing[0],
+        return Bound{reinterpret_cast<const V4*>(lds), start[0], spacing[0], T(1) / spacing[0],
                      static_cast<T>(knots - 2)};
     }
 };
