@@ -97,10 +97,23 @@ int ndn_update(int dtype, const void* positions, const void* cell, double cutoff
                void* reuse, int32_t* rebuild, int32_t* rebuild_count,
                const ndn_neighbor_buffers* buffers, ndn_stream_t stream);
 
+/* For the host code of a first frame, one readback each (no counterpart in the reference, which
+ * reads its cell and a reduction of its positions apart, _neighbor_list.py:87-113,234-272):
+ * inspect_frame puts the cell's edges in found [0..2] and the number of coordinates that are not
+ * finite in found [3] (double, device, zero before the call); count_totals puts a count's pairs in
+ * totals [0] and its full list's entries, if it keeps one, in totals [1] (device, zero before). */
+int ndn_inspect_frame(int dtype, const void* positions, const void* cell, int64_t num_atoms,
+                      double* found, ndn_stream_t stream);
+int ndn_count_totals(const ndn_neighbor_buffers* buffers, int64_t* totals, ndn_stream_t stream);
+
 /* Wrap positions [N, 3] into [0, L) per axis, adding lattice crossings to images [N, 3] int64
  * (images may be NULL). Replaces space.wrap (space.py:22-38); out may alias positions. */
 int ndn_wrap(int dtype, const void* positions, const void* cell, int64_t num_atoms, void* out,
              int64_t* images, ndn_stream_t stream);
+
+/* ndn_wrap over frames: positions [F, N, 3] into cells [F, 3] (images [F, N, 3] or NULL). */
+int ndn_wrap_frames(int dtype, const void* positions, const void* cells, int64_t frames,
+                    int64_t num_atoms, void* out, int64_t* images, ndn_stream_t stream);
 
 /* ---- pair potentials -------------------------------------------------------------------- */
 

@@ -983,14 +983,52 @@ __global__ void __launch_bounds__(kBlock) total_pad_commit_kernel(
     if (gid == 0) ++rebuild_count[0];
 }
 
+// What a first frame's host code reads: the cell's edges in found [0..2] and how many coordinates
+// are not finite in found [3] (found zero before the launch).
+template <typename T>
+__global__ void __launch_bounds__(kBlock) inspect_frame_kernel(const T* __restrict__ positions,
+                                                               const T* __restrict__ cell,
+                                                               std::int64_t count,
+                                                               double* __restrict__ found)
+{
+    const std::int64_t first = static_cast<std::int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    const std::int64_t stride = static_cast<std::int64_t>(gridDim.x) * blockDim.x;
+    int bad = 0;
+    for (std::int64_t k = first; k < count; k += stride) bad += !isfinite(positions[k]);
+    if (bad != 0) unsafeAtomicAdd(found + 3, static_cast<double>(bad));
+    if (first < 3) found[first] = static_cast<double>(cell[first]);
+}
+
+// The pairs of a count in totals [0], as 64-bit sums, and the entries of its full list in
+// totals [1] (totals zero before the launch).
+__global__ void __launch_bounds__(kBlock) count_totals_kernel(
+    const index_t* __restrict__ pair_counts, std::int64_t num_atoms,
+    const index_t* __restrict__ full_slices, std::int64_t num_slices,
+    unsigned long long* __restrict__ totals)
+{
+    __shared__ unsigned long long shared[16];
+    const std::int64_t first = static_cast<std::int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    const std::int64_t stride = static_cast<std::int64_t>(gridDim.x) * blockDim.x;
+    unsigned long long sum = 0;
+    for (std::int64_t k = first; k < num_atoms; k += stride)
+        sum += static_cast<unsigned long long>(pair_counts[k]);
+    sum = block_sum(sum, shared);
+    if (threadIdx.x == 0 && sum != 0) atomicAdd(totals, sum);
+    if (first == 0 && full_slices != nullptr)
+        totals[1] = static_cast<unsigned long long>(full_slices[num_slices]);
+}
+
+// Coordinates [frames, N, 3] into the frames' cells [frames, 3], `per_frame` = 3N coordinates to a
+// frame.
 template <typename T>
 __global__ void __launch_bounds__(kBlock) wrap_kernel(const T* positions, const T* __restrict__ cell,
-                                                      std::int64_t count, T* out,
-                                                      std::int64_t* __restrict__ images)
+                                                      std::int64_t count, std::int64_t per_frame,
+                                                      T* out, std::int64_t* __restrict__ images)
 {
     const std::int64_t index = static_cast<std::int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
     if (index >= count) return;
-    const T length = cell[index % 3];
+    const std::int64_t frame = count == per_frame ? 0 : index / per_frame;
+    const T length = cell[3 * frame + index % 3];
     const T v = positions[index];
     T k = floor(v / length);
     T w = v - k * length;
@@ -1347,26 +1385,67 @@ int ndn_update(int dtype, const void* positions, const void* cell, double cutoff
                                stream);
 }
 
-int ndn_wrap(int dtype, const void* positions, const void* cell, int64_t num_atoms, void* out,
-             int64_t* images, ndn_stream_t stream)
+int ndn_inspect_frame(int dtype, const void* positions, const void* cell, int64_t num_atoms,
+                      double* found, ndn_stream_t stream)
 {
-    NDN_REQUIRE(positions && cell && out, "positions, cell and out must not be null");
-    NDN_REQUIRE(num_atoms >= 0, "N must be nonnegative");
-    if (num_atoms == 0) return NDN_OK;
+    NDN_REQUIRE(positions && cell && found, "a buffer is null");
+    NDN_REQUIRE(num_atoms >= 1 && num_atoms <= INT32_MAX, "N must satisfy 1 <= N < 2**31");
     const std::int64_t count = 3 * num_atoms;
+    const unsigned blocks = std::min(blocks_for(count), kPadBlocks);
+    if (dtype == NDN_F32)
+        inspect_frame_kernel<float><<<blocks, kBlock, 0, stream>>>(
+            static_cast<const float*>(positions), static_cast<const float*>(cell), count, found);
+    else
+    {
+        NDN_REQUIRE(dtype == NDN_F64, "dtype must be NDN_F32 or NDN_F64");
+        inspect_frame_kernel<double><<<blocks, kBlock, 0, stream>>>(
+            static_cast<const double*>(positions), static_cast<const double*>(cell), count, found);
+    }
+    NDN_LAUNCHED("inspect_frame");
+    return NDN_OK;
+}
+
+int ndn_count_totals(const ndn_neighbor_buffers* buffers, int64_t* totals, ndn_stream_t stream)
+{
+    const int checked = check_buffers(buffers);
+    if (checked != NDN_OK) return checked;
+    NDN_REQUIRE(totals != nullptr, "totals must not be null");
+    const std::int64_t n = buffers->num_atoms;
+    const bool full = buffers->full_index != nullptr;
+    count_totals_kernel<<<std::min(blocks_for(n), kPadBlocks), kBlock, 0, stream>>>(
+        buffers->pair_counts, n, full ? buffers->full_slices : nullptr, (n + kWave - 1) / kWave,
+        reinterpret_cast<unsigned long long*>(totals));
+    NDN_LAUNCHED("count_totals");
+    return NDN_OK;
+}
+
+int ndn_wrap_frames(int dtype, const void* positions, const void* cells, int64_t frames,
+                    int64_t num_atoms, void* out, int64_t* images, ndn_stream_t stream)
+{
+    NDN_REQUIRE(positions && cells && out, "positions, cell and out must not be null");
+    NDN_REQUIRE(frames >= 0 && num_atoms >= 0, "N must be nonnegative");
+    const std::int64_t each = 3 * num_atoms;
+    const std::int64_t count = frames * each;
+    if (count == 0) return NDN_OK;
     if (dtype == NDN_F32)
         wrap_kernel<float><<<blocks_for(count), kBlock, 0, stream>>>(
-            static_cast<const float*>(positions), static_cast<const float*>(cell), count,
+            static_cast<const float*>(positions), static_cast<const float*>(cells), count, each,
             static_cast<float*>(out), images);
     else
     {
         NDN_REQUIRE(dtype == NDN_F64, "dtype must be NDN_F32 or NDN_F64");
         wrap_kernel<double><<<blocks_for(count), kBlock, 0, stream>>>(
-            static_cast<const double*>(positions), static_cast<const double*>(cell), count,
+            static_cast<const double*>(positions), static_cast<const double*>(cells), count, each,
             static_cast<double*>(out), images);
     }
     NDN_LAUNCHED("wrap");
     return NDN_OK;
+}
+
+int ndn_wrap(int dtype, const void* positions, const void* cell, int64_t num_atoms, void* out,
+             int64_t* images, ndn_stream_t stream)
+{
+    return ndn_wrap_frames(dtype, positions, cell, 1, num_atoms, out, images, stream);
 }
 
 }  // extern "C"

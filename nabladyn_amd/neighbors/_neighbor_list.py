@@ -126,24 +126,44 @@ class _Plan:
 
     @staticmethod
     def of(positions: Tensor, cell: Tensor, settings: _Settings) -> "_Plan":
-        """Syncs with the host (the cell, and whether every coordinate is finite)."""
-        lengths = tuple(float(v) for v in cell.tolist())
+        """Syncs with the host once (the cell, and whether every coordinate is finite)."""
+        n = positions.shape[0]
+        found = torch.zeros(4, dtype=torch.float64, device=positions.device)
+        _native.call("inspect_frame", _native.dtype_tag(positions.dtype), _native.ptr(positions),
+                     _native.ptr(cell), _native.ctypes.c_int64(n), _native.ptr(found),
+                     _native.stream(positions.device))
+        *lengths, bad = found.tolist()
         if not all(math.isfinite(v) and v > 2 * settings.cutoff for v in lengths):
             raise ValueError("every cell length must be finite and above twice the cutoff")
-        if not bool(torch.isfinite(positions).all()):
+        if bad:
             raise ValueError("positions must be finite")
-        dims = tuple(grid_dims(list(lengths), settings.radius, positions.dtype))
-        n = positions.shape[0]
+        dims = tuple(grid_dims(lengths, settings.radius, positions.dtype))
         if math.prod(dims) >= _INT32_MAX:
             raise ValueError("the grid must have fewer than 2**31 - 1 bins")
-        scan = max(_ops.scan_temp_bytes(positions, math.prod(dims) + 1),
-                   _ops.scan_temp_bytes(positions, n))
-        return _Plan(lengths, dims, n, scan)
+        scan = _ops.scan_temp_bytes(positions, max(math.prod(dims) + 1, n))
+        return _Plan(tuple(lengths), dims, n, scan)
+
+
+def _cut(block: Tensor, sizes: dict[str, tuple[int, torch.dtype]]) -> dict[str, Tensor]:
+    """Tensors of the given lengths and dtypes cut from a block of bytes, each starting at a
+    multiple of 256 bytes."""
+    out, start = {}, 0
+    for name, (length, dtype) in sizes.items():
+        end = start + length * dtype.itemsize
+        out[name] = block[start:end].view(dtype)
+        start = -(-end // 256) * 256
+    return out
+
+
+def _block_bytes(sizes: dict[str, tuple[int, torch.dtype]]) -> int:
+    return sum(-(-length * dtype.itemsize // 256) * 256 for length, dtype in sizes.values())
 
 
 class _Device:
     """The list's device tensors: the operators' buffers (one table, in argument order), the
-    reuse rule's tensors, and the full list when one is kept."""
+    reuse rule's tensors, and the full list when one is kept. Those that start at zero, and those
+    that start with what the plan says, are cut from one allocation each: a list of a small frame
+    is made in a few launches and copies."""
 
     def __init__(self, plan: _Plan, positions: Tensor, settings: _Settings):
         device, dtype, n = positions.device, positions.dtype, plan.num_atoms
@@ -151,33 +171,53 @@ class _Device:
         per_atom = lambda: torch.empty(n, **ints)  # noqa: E731
         bins = plan.num_bins + 1
         words = n * ((n + 31) // 32) if plan.all_pairs else 0
+        zeros = {"bin_counts": (bins, torch.int32), "scan_temp": (plan.scan_bytes, torch.uint8),
+                 "pair_total": (1, torch.int32), "status": (2, torch.int32),
+                 "bits": (words, torch.int32), "parameters": (4, dtype),
+                 "rebuild": (1, torch.int32)}
+        if settings.full:
+            zeros["counts"] = (n, torch.int32)
+            zeros["slices"] = ((n + _ROWS_PER_SLICE - 1) // _ROWS_PER_SLICE + 1, torch.int32)
+        zero = _cut(torch.zeros(_block_bytes(zeros), dtype=torch.uint8, device=device), zeros)
+        said = {"dims": (3, torch.int32), "limits": (3, torch.int32), "widths": (3, dtype),
+                "rebuild_count": (1, torch.int32)}
+        host = torch.zeros(_block_bytes(said), dtype=torch.uint8)
+        for name, values in _cut(host, said).items():
+            values.copy_(torch.tensor({
+                "dims": plan.dims, "limits": plan.dims, "rebuild_count": (1,),
+                "widths": [length / count for length, count in zip(plan.lengths, plan.dims)],
+            }[name], dtype=values.dtype))
+        said = _cut(host.to(device), said)
         table = {
-            "dims": torch.tensor(plan.dims, **ints),
-            "widths": torch.tensor([length / count for length, count in zip(plan.lengths, plan.dims)],
-                                   dtype=dtype, device=device),
+            "dims": said["dims"],
+            "widths": said["widths"],
             "atom_bin": per_atom(),
-            "bin_counts": torch.zeros(bins, **ints),
+            "bin_counts": zero["bin_counts"],
             "bin_offsets": torch.empty(bins, **ints),
             "unordered_ids": per_atom(),
             "sorted_ids": per_atom(),
             "sorted_positions": torch.empty((n, 3), dtype=dtype, device=device),
-            "scan_temp": torch.zeros(plan.scan_bytes, dtype=torch.uint8, device=device),
+            "scan_temp": zero["scan_temp"],
             "pair_counts": per_atom(),
             "pair_offsets": per_atom(),
-            "pair_total": torch.zeros(1, **ints),
-            "status": torch.zeros(2, **ints),
+            "pair_total": zero["pair_total"],
+            "status": zero["status"],
             "pairs": torch.empty((2, 1), **ints),  # sized once the pairs are counted
-            "bits": torch.zeros(words, **ints),
+            "bits": zero["bits"],
         }
         assert tuple(table) == _ops.BUFFER_NAMES
         self.buffers = table
         self.full = None
         if settings.full:
             self.full = {
-                "counts": torch.zeros(n, **ints),
-                "slices": torch.zeros((n + _ROWS_PER_SLICE - 1) // _ROWS_PER_SLICE + 1, **ints),
-                "index": torch.zeros(1, **ints),  # sized once the pairs are counted
+                "counts": zero["counts"],
+                "slices": zero["slices"],
+                "index": torch.empty(1, **ints),  # sized once the pairs are counted
             }
+        # the reuse rule's grid limits, scratch, flag and build count, and after a first build
+        # (``start_reuse``) its frame
+        self._rule = {"limits": said["limits"], "parameters": zero["parameters"],
+                      "rebuild": zero["rebuild"], "rebuild_count": said["rebuild_count"]}
         self.reuse = None
         self.native = None
 
@@ -188,18 +228,11 @@ class _Device:
     def bind(self, positions: Tensor) -> None:
         self.native = _ops.native_buffers(positions, self.buffers, self.full)
 
-    def start_reuse(self, wrapped: Tensor, cell: Tensor, dims) -> None:
-        """The reuse rule's state after a first build: its frame, its grid as the limits of
-        later grids, the rule's scratch, the flag and the build count (1)."""
-        ints = {"dtype": torch.int32, "device": wrapped.device}
-        self.reuse = {
-            "reference_positions": wrapped.clone(),
-            "reference_cell": cell.clone(),
-            "limits": torch.tensor(dims, **ints),
-            "parameters": torch.zeros(4, dtype=wrapped.dtype, device=wrapped.device),
-            "rebuild": torch.zeros(1, **ints),
-            "rebuild_count": torch.ones(1, **ints),
-        }
+    def start_reuse(self, wrapped: Tensor, cell: Tensor) -> None:
+        """The reuse rule's state after a first build: its frame (``wrapped`` is the list's from
+        here on), its grid as the limits of later grids, the rule's scratch, the flag and the
+        build count (1)."""
+        self.reuse = {"reference_positions": wrapped, "reference_cell": cell.clone(), **self._rule}
 
 
 def _message_invalid_cell(nl, needed):
@@ -301,32 +334,40 @@ class NeighborList:
         cell, and ``ValueError`` when the grid or the pairs do not fit int32.
         """
         _check_frame(positions, cell)
-        settings = self._settings
-        plan = _Plan.of(positions, cell, settings)
-        dev = _Device(plan, positions, settings)
-        cell = cell.detach().contiguous()
-        wrapped, _ = space.wrap(positions.detach(), cell)
-        # count, size what the count fixes, fill
-        _ops.count_first_frame(wrapped, cell, self.radius, dev.buffers, dev.full)
-        totals = [dev.buffers["pair_counts"].sum(dtype=torch.int64)]
-        if dev.full is not None:
-            totals.append(dev.full["slices"][-1].to(torch.int64))
-        counts = [int(v) for v in torch.stack(totals).tolist()]
-        ints = {"dtype": torch.int32, "device": positions.device}
-        dev.buffers["pairs"] = torch.empty(
-            (2, pair_capacity_for(counts[0], settings.multiplier)), **ints)
-        if dev.full is not None:
-            dev.full["index"] = torch.zeros(
-                pair_capacity_for(counts[1], settings.multiplier, _ROWS_PER_SLICE), **ints)
-        _ops.fill_first_frame(wrapped, cell, self.radius, dev.buffers, dev.full)
-        dev.start_reuse(wrapped, cell, plan.dims)
-        dev.bind(wrapped)
+        with torch.cuda.device(positions.device):
+            dev = self._build_first(positions.detach().contiguous(), cell.detach().contiguous())
         self._device = dev
         # the list fails as a whole until every inner list is built
         self._failure = "an inner list was not allocated"
         for inner in self._inner:
             inner.allocate(positions, cell)
         self._failure = None
+
+    def _build_first(self, positions: Tensor, cell: Tensor) -> _Device:
+        """Count, size what the count fixes, fill: two readbacks of a few numbers."""
+        settings = self._settings
+        plan = _Plan.of(positions, cell, settings)
+        dev = _Device(plan, positions, settings)
+        wrapped = space.wrapped(positions, cell)
+        dev.bind(wrapped)
+        stream = _native.stream(wrapped.device)
+        frame = (_native.dtype_tag(wrapped.dtype), _native.ptr(wrapped), _native.ptr(cell),
+                 _native.ctypes.c_double(self.radius))
+        _native.call("count_first_frame", *frame, _native.ctypes.byref(dev.native), stream)
+        totals = torch.zeros(2, dtype=torch.int64, device=positions.device)
+        _native.call("count_totals", _native.ctypes.byref(dev.native), _native.ptr(totals), stream)
+        pairs, entries = totals.tolist()
+        ints = {"dtype": torch.int32, "device": positions.device}
+        dev.buffers["pairs"] = torch.empty((2, pair_capacity_for(pairs, settings.multiplier)),
+                                           **ints)
+        if dev.full is not None:
+            # entries past a row's count are never read
+            dev.full["index"] = torch.empty(
+                pair_capacity_for(entries, settings.multiplier, _ROWS_PER_SLICE), **ints)
+        dev.start_reuse(wrapped, cell)
+        dev.bind(wrapped)
+        _native.call("fill_first_frame", *frame, _native.ctypes.byref(dev.native), stream)
+        return dev
 
     def update(self, positions: Tensor, cell: Tensor) -> None:
         """Reuse the pairs for positions [N, 3] in the cell [3], or rebuild them.
@@ -340,7 +381,7 @@ class NeighborList:
         if (positions.shape, positions.dtype, positions.device) != (
                 sorted_positions.shape, sorted_positions.dtype, sorted_positions.device):
             raise ValueError("positions must match the allocated shape, dtype and device")
-        wrapped, _ = space.wrap(positions.detach(), cell.detach())
+        wrapped = space.wrapped(positions, cell)
         self._update_wrapped(wrapped, cell.detach().contiguous())
         self._check_status()
 

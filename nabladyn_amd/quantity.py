@@ -94,7 +94,7 @@ def _bind(energy_fn, energy: bool, forces: bool, virial: bool):
         def evaluate(positions: Tensor, cell: Tensor, pairs: NeighborPairs):
             if wraps:
                 model._check_inputs(positions, cell, pairs)
-                positions, _ = space.wrap(positions.detach(), cell)
+                positions = space.wrapped(positions, cell)
             results = _evaluate(model, positions, cell, pairs, energy=energy, forces=forces,
                                 virial=virial)
             return tuple(v for v in results if v is not None)

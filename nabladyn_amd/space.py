@@ -69,6 +69,37 @@ def wrap(positions: Tensor, cell: Tensor) -> tuple[Tensor, Tensor]:
     return _Wrap.apply(positions, cell)
 
 
+def wrapped(positions: Tensor, cell: Tensor) -> Tensor:
+    """``wrap``'s positions alone, with no derivatives and no crossings to clear and count: one
+    launch. For callers that use neither."""
+    _native.require_gpu(positions, "positions")
+    if positions.dim() != 2 or positions.shape[-1] != 3 or cell.shape != (3,):
+        raise ValueError("wrap takes positions [N, 3] and a cell [3]")
+    x = positions.detach().contiguous()
+    out = torch.empty_like(x)
+    wrap_into(x, cell.detach().to(x.dtype).contiguous(), out)
+    return out
+
+
+def wrapped_frames(positions: Tensor, cells: Tensor) -> Tensor:
+    """``wrapped`` of frames [F, N, 3] in cells [F, 3] (those past the frames unused), one
+    launch."""
+    _native.require_gpu(positions, "positions")
+    if (positions.dim() != 3 or positions.shape[-1] != 3 or cells.dim() != 2
+            or cells.shape[0] < positions.shape[0] or cells.shape[1] != 3
+            or cells.device != positions.device):
+        raise ValueError("wrap takes positions [F, N, 3] and cells [F, 3] on one device")
+    x = positions.detach().contiguous()
+    cells = cells.detach().to(x.dtype).contiguous()
+    out = torch.empty_like(x)
+    _native.call(
+        "wrap_frames", _native.dtype_tag(x.dtype), _native.ptr(x), _native.ptr(cells),
+        _native.ctypes.c_int64(x.shape[0]), _native.ctypes.c_int64(x.shape[1]), _native.ptr(out),
+        None, _native.stream(x.device),
+    )
+    return out
+
+
 def wrap_into(positions: Tensor, cell: Tensor, out: Tensor, images: Tensor | None = None) -> None:
     """Wrap positions [N, 3] into ``out`` (may be ``positions``), adding crossings to ``images``.
 

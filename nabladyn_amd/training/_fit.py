@@ -59,8 +59,7 @@ def pair_stack(positions: Tensor, cells: Tensor, cutoff: float) -> Tensor:
     """
     frames, atoms = positions.shape[:2]
     cells = cells.detach().contiguous()
-    wrapped = torch.stack([space.wrap(positions[f].detach(), cells[f])[0]
-                           for f in range(frames)]).contiguous()
+    wrapped = space.wrapped_frames(positions, cells)
     densest = 0
     while True:
         counter, totals, status = _frame_totals(wrapped, cells, cutoff, densest)
@@ -158,8 +157,7 @@ def _prepare(model: Potential, data: Dataset, channels: tuple[str, ...]) -> _Pre
         return value.to(device=model.device, dtype=model.dtype)
 
     positions, cells = moved(data.positions), moved(data.cells)
-    positions = torch.stack([space.wrap(positions[f], cells[f])[0]
-                             for f in range(positions.shape[0])]).contiguous()
+    positions = space.wrapped_frames(positions, cells)
     stacks = tuple(pair_stack(positions, cells, cutoff) for cutoff in model._list_cutoffs)
     rows = None
     if model._fused:
