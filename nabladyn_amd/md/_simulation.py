@@ -143,10 +143,12 @@ def brick_shapes(dims: list[int], num_atoms: int, dtype: torch.dtype, reserve: i
 
 def potential_reserve(model) -> int:
     """Halo positions' worth of LDS the force kernel stages for the model beside the halo: a
-    one-type table's segments, two 4-vectors each (the LDS budget of two blocks per CU holds
-    both)."""
-    from ..potential import Tabulated
+    one-type table's segments, two 4-vectors each, or the coefficients of up to 8 types' pairs,
+    one each (the LDS budget of two blocks per CU holds both)."""
+    from ..potential import LennardJones, Tabulated
 
+    if isinstance(model, LennardJones) and 1 < model._num_types <= 8:
+        return model._num_types ** 2
     if isinstance(model, Tabulated) and model.table.shape[0] == 1:
         return 2 * (int(model.table.shape[1]) - 1)
     return 0
