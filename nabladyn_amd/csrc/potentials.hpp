@@ -11,8 +11,10 @@
 
 namespace ndn {
 
-// 1 / value: the hardware reciprocal in fp32 (1 ulp), a division in fp64. For factors that only
-// scale a force.
+// 1 / value: the hardware reciprocal in fp32 (1 ulp); in fp64 the hardware's estimate with two
+// Newton steps, whose result is the correctly rounded one but next to a rounding boundary, in half
+// the instructions of a division (which also scales operands near the ends of the range). For
+// factors that only scale a force. Zero gives NaN in fp64, where its caller's terms are NaN too.
 template <typename T>
 __device__ __forceinline__ T reciprocal(T value);
 template <>
@@ -23,11 +25,13 @@ __device__ __forceinline__ float reciprocal<float>(float value)
 template <>
 __device__ __forceinline__ double reciprocal<double>(double value)
 {
-    return 1.0 / value;
+    double y = __builtin_amdgcn_rcp(value);
+    y = __builtin_fma(__builtin_fma(-value, y, 1.0), y, y);
+    return __builtin_fma(__builtin_fma(-value, y, 1.0), y, y);
 }
 
-// sqrt(x), correctly rounded: in fp32 the hardware's reciprocal square root with two coupled
-// Newton steps and a last one on the remainder (P. W. Markstein, "Computation of elementary
+// sqrt(x), correctly rounded: the hardware's reciprocal square root with a coupled Newton step (two
+// in fp64) and a last one on the remainder (P. W. Markstein, "Computation of elementary
 // functions on the IBM RISC System/6000 processor", 1990), without the scaling that a library's
 // root does for results near the ends of the range: squared distances are far from them, and one
 // that is not takes the hardware's root.
@@ -36,7 +40,16 @@ __device__ __forceinline__ T pair_distance(T x);
 template <>
 __device__ __forceinline__ double pair_distance<double>(double x)
 {
-    return sqrt(x);
+    const double y = __builtin_amdgcn_rsq(x);
+    double g = x * y, h = 0.5 * y;
+    double r = __builtin_fma(-h, g, 0.5);
+    g = __builtin_fma(g, r, g);
+    h = __builtin_fma(h, r, h);
+    r = __builtin_fma(-h, g, 0.5);
+    g = __builtin_fma(g, r, g);
+    h = __builtin_fma(h, r, h);
+    g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
+    return x > 1e-200 ? g : __builtin_amdgcn_sqrt(x);
 }
 template <>
 __device__ __forceinline__ float pair_distance<float>(float x)
@@ -50,13 +63,13 @@ __device__ __forceinline__ float pair_distance<float>(float x)
     return x > 1e-30f ? g : __builtin_amdgcn_sqrtf(x);
 }
 
-// 1 / x: the hardware reciprocal with one Newton step in fp32, a division in fp64.
+// 1 / x: the hardware reciprocal with one Newton step in fp32, two in fp64.
 template <typename T>
 __device__ __forceinline__ T refined_reciprocal(T x);
 template <>
 __device__ __forceinline__ double refined_reciprocal<double>(double x)
 {
-    return 1.0 / x;
+    return reciprocal(x);
 }
 template <>
 __device__ __forceinline__ float refined_reciprocal<float>(float x)
@@ -128,11 +141,15 @@ struct Table
 
     __device__ __forceinline__ void eval(int row_index, T r2, T& u, T& fs) const
     {
-        // r and the knot coordinate with the reference's own operations, each correctly
-        // rounded (sqrt, subtract, divide), so t and the segment are the reference's bits
-        const T r = sqrt(r2);
+        // r and the knot coordinate are the reference's: its square root, subtraction and
+        // division, each correctly rounded (pair_distance; the quotient is a product with 1/h
+        // corrected by its remainder), so t and the segment are the reference's bits
+        const T r = pair_distance(r2);
         const T h = spacing[row_index];
-        const T x = (r - start[row_index]) / h;
+        const T inverse_h = refined_reciprocal(h);
+        const T offset = r - start[row_index];
+        const T q = offset * inverse_h;
+        const T x = fma(fma(-q, h, offset), inverse_h, q);
         T segment = floor(x);
         segment = segment < T(0) ? T(0) : (segment > T(knots - 2) ? T(knots - 2) : segment);
         const T t = x - segment;
@@ -147,8 +164,8 @@ struct Table
         const bool below = t < T(0);
         u = cubic + (below ? T(0.5) * a * t : T(0));
         const T du_dt = below ? T(0.5) * a : T(0.5) * (a + s * (T(2) * b + T(3) * s * c));
-        // 1/h and 1/r only scale the force: hardware reciprocals
-        fs = -(du_dt * reciprocal(h)) * reciprocal(r);
+        // 1/r only scales the force: the hardware's reciprocal
+        fs = -(du_dt * inverse_h) * reciprocal(r);
     }
 };
 
