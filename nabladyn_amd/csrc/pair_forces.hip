@@ -188,21 +188,6 @@ __device__ __forceinline__ void stage_in_block(Pot& pot, unsigned char* lds)
 
 // ---- half-list schedule ---------------------------------------------------------------------
 
-// The sum of `value` over each run of lanes with the same key (a run starts where the key
-// changes), left in the run's last lane; `start` is the run's first lane. Equal keys apart are
-// separate runs.
-template <typename T>
-__device__ __forceinline__ T run_sum(T value, int lane, int start)
-{
-#pragma unroll
-    for (int offset = 1; offset < kWave; offset <<= 1)
-    {
-        const T other = __shfl_up(value, offset, kWave);
-        if (lane - offset >= start) value += other;
-    }
-    return value;
-}
-
 //
 // Frames of one system (training stacks) take blockIdx.y as the frame: its positions [N, 3],
 // cell [3], pairs [2, C], forces [N, 3] and the grid's partial slots follow the previous frame's.
@@ -276,34 +261,7 @@ __global__ void __launch_bounds__(kBlock) half_list_kernel(
         }
         if (kForces)
         {
-            if (inside)
-            {
-                unsafeAtomicAdd(forces + 3LL * j, -fx);
-                unsafeAtomicAdd(forces + 3LL * j + 1, -fy);
-                unsafeAtomicAdd(forces + 3LL * j + 2, -fz);
-            }
-            // runs of the same first atom (padding and unlisted columns key -1)
-            const index_t key = listed ? i : -1;
-            const index_t before = __shfl_up(key, 1, kWave);
-            const bool head = lane == 0 || before != key;
-            int start = head ? lane : 0;
-#pragma unroll
-            for (int offset = 1; offset < kWave; offset <<= 1)
-            {
-                const int other = __shfl_up(start, offset, kWave);
-                if (lane >= offset && other > start) start = other;
-            }
-            const T sx = run_sum(fx, lane, start);
-            const T sy = run_sum(fy, lane, start);
-            const T sz = run_sum(fz, lane, start);
-            const int next_start = __shfl_down(start, 1, kWave);
-            const bool tail = lane == kWave - 1 || next_start != start;
-            if (tail && key >= 0)
-            {
-                unsafeAtomicAdd(forces + 3LL * key, sx);
-                unsafeAtomicAdd(forces + 3LL * key + 1, sy);
-                unsafeAtomicAdd(forces + 3LL * key + 2, sz);
-            }
+            add_pair_forces(forces, listed ? i : -1, inside ? j : -1, fx, fy, fz, lane);
         }
     }
     store_partials<kVirial>(static_cast<double>(energy), w, shared, partials);

@@ -59,6 +59,65 @@ struct PotentialView
     Table<T> table;
 };
 
+// The sum of `value` over each run of lanes with the same key (a run starts where the key
+// changes), left in the run's last lane; `start` is the run's first lane. Equal keys apart are
+// separate runs.
+template <typename T>
+__device__ __forceinline__ T run_sum(T value, int lane, int start)
+{
+#pragma unroll
+    for (int offset = 1; offset < kWave; offset <<= 1)
+    {
+        const T other = __shfl_up(value, offset, kWave);
+        if (lane - offset >= start) value += other;
+    }
+    return value;
+}
+
+// Adds a wave's pair forces to both atoms, f to `i` and -f to `j` (a negative id takes nothing),
+// for lanes that walk consecutive columns of a half list; every lane of the wave takes part.
+//
+// What bounds it is the atomics, which meet in memory past the XCDs' own L2s, each a request of
+// its own: 13 million of them, of a lane per pair, held 100,000 atoms at 0.67 ms. So the forces of
+// the first atom are summed over its run of columns before they go out, and those of the second
+// go out as its three components in neighboring lanes, which a request takes together.
+template <typename T>
+__device__ __forceinline__ void add_pair_forces(T* __restrict__ forces, index_t i, index_t j, T fx,
+                                                T fy, T fz, int lane)
+{
+#pragma unroll
+    for (int turn = 0; turn < 3; ++turn)
+    {
+        const int component = kWave * turn + lane;
+        const int from = component / 3, axis = component - 3 * from;
+        const index_t atom = __shfl(j, from, kWave);
+        const T x = __shfl(fx, from, kWave), y = __shfl(fy, from, kWave),
+                z = __shfl(fz, from, kWave);
+        const T value = axis == 0 ? x : (axis == 1 ? y : z);
+        if (atom >= 0) unsafeAtomicAdd(forces + 3LL * atom + axis, -value);
+    }
+    const index_t before = __shfl_up(i, 1, kWave);
+    const bool head = lane == 0 || before != i;
+    int start = head ? lane : 0;
+#pragma unroll
+    for (int offset = 1; offset < kWave; offset <<= 1)
+    {
+        const int other = __shfl_up(start, offset, kWave);
+        if (lane >= offset && other > start) start = other;
+    }
+    const T sx = run_sum(fx, lane, start);
+    const T sy = run_sum(fy, lane, start);
+    const T sz = run_sum(fz, lane, start);
+    const int next_start = __shfl_down(start, 1, kWave);
+    const bool tail = lane == kWave - 1 || next_start != start;
+    if (tail && i >= 0)
+    {
+        unsafeAtomicAdd(forces + 3LL * i, sx);
+        unsafeAtomicAdd(forces + 3LL * i + 1, sy);
+        unsafeAtomicAdd(forces + 3LL * i + 2, sz);
+    }
+}
+
 // Writes this block's energy and virial sums to partials[8 * blockIdx.x ...].
 template <bool kVirial, typename T>
 __device__ __forceinline__ void store_partials(double energy, const T* w, double* shared,

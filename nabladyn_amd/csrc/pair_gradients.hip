@@ -132,8 +132,8 @@ __device__ __forceinline__ bool listed_pair(index_t i, index_t j, index_t num_at
 
 constexpr int kStrainedSlot = 16;  // doubles per block: E, W[9], padding
 
-// E, F and W at a nonzero strain over a half list: a lane per column, both atoms' forces added
-// with atomics.
+// E, F and W at a nonzero strain over a half list: a lane per column, a wave's forces added
+// together (add_pair_forces).
 template <typename T, class Pot>
 __global__ void __launch_bounds__(kBlock) strained_pairs_kernel(
     const T* __restrict__ positions, const T* __restrict__ cell, const index_t* __restrict__ pairs,
@@ -142,33 +142,47 @@ __global__ void __launch_bounds__(kBlock) strained_pairs_kernel(
 {
     __shared__ double shared[16];
     const Strain<T> strain = read_strain(strain_matrix);
+    const int lane = lane_id();
     double energy = 0;
     double w[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
     const std::int64_t stride = static_cast<std::int64_t>(gridDim.x) * blockDim.x;
-    for (std::int64_t column = static_cast<std::int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-         column < capacity; column += stride)
+    for (std::int64_t first =
+             static_cast<std::int64_t>(blockIdx.x) * blockDim.x + threadIdx.x - lane;
+         first < capacity; first += stride)
     {
-        const index_t i = pairs[column];
-        const index_t j = pairs[capacity + column];
-        if (!listed_pair(i, j, num_atoms)) continue;
-        T d[3], dp[3];
-        const T r2 = pair_geometry<T, true>(positions, cell, i, j, strain, d, dp);
-        if (!(r2 < cutoff_squared)) continue;
-        T u, fs;
-        pot.eval(pot.row(i, j), r2, u, fs);
-        energy += static_cast<double>(u);
-        for (int b = 0; b < 3; ++b)
+        const std::int64_t column = first + lane;
+        index_t i = -1, j = -1;
+        if (column < capacity)
         {
-            const T back = (strain.e[b] * dp[0] + strain.e[3 + b] * dp[1]) + strain.e[6 + b] * dp[2];
-            const T g = fs * (dp[b] + back);
-            if (forces != nullptr)
+            i = pairs[column];
+            j = pairs[capacity + column];
+        }
+        const bool listed = listed_pair(i, j, num_atoms);
+        T g[3] = {0, 0, 0};
+        bool inside = false;
+        if (listed)
+        {
+            T d[3], dp[3];
+            const T r2 = pair_geometry<T, true>(positions, cell, i, j, strain, d, dp);
+            inside = r2 < cutoff_squared;
+            if (inside)
             {
-                unsafeAtomicAdd(forces + 3LL * i + b, g);
-                unsafeAtomicAdd(forces + 3LL * j + b, -g);
+                T u, fs;
+                pot.eval(pot.row(i, j), r2, u, fs);
+                energy += static_cast<double>(u);
+                for (int b = 0; b < 3; ++b)
+                {
+                    const T back =
+                        (strain.e[b] * dp[0] + strain.e[3 + b] * dp[1]) + strain.e[6 + b] * dp[2];
+                    g[b] = fs * (dp[b] + back);
+                }
+                for (int a = 0; a < 3; ++a)
+                    for (int b = 0; b < 3; ++b)
+                        w[3 * a + b] += static_cast<double>(fs * dp[a] * d[b]);
             }
         }
-        for (int a = 0; a < 3; ++a)
-            for (int b = 0; b < 3; ++b) w[3 * a + b] += static_cast<double>(fs * dp[a] * d[b]);
+        if (forces != nullptr)
+            add_pair_forces(forces, listed ? i : -1, inside ? j : -1, g[0], g[1], g[2], lane);
     }
     const double e = block_sum(energy, shared);
     double v[9];
