@@ -172,6 +172,28 @@ __device__ __forceinline__ V block_sum(V value, V* shared)
     return sum;
 }
 
+// The block's sums of N values behind one barrier: thread k < N returns the k-th, in the order of
+// block_sum (any other thread a meaningless value). `shared` holds 16 N values, which no other use
+// of it may touch before a barrier.
+template <int N, typename V>
+__device__ __forceinline__ V block_sums(V (&values)[N], V* shared)
+{
+    const int lane = lane_id();
+    const int wave = threadIdx.x / kWave;
+    const int waves = blockDim.x / kWave;
+#pragma unroll
+    for (int k = 0; k < N; ++k)
+    {
+        values[k] = wave_sum(values[k]);
+        if (lane == 0) shared[16 * k + wave] = values[k];
+    }
+    __syncthreads();
+    V sum = 0;
+    if (threadIdx.x < N)
+        for (int w = 0; w < waves; ++w) sum += shared[16 * threadIdx.x + w];
+    return sum;
+}
+
 // ---- C-ABI error plumbing -------------------------------------------------------------------
 
 void set_error(const std::string& message);

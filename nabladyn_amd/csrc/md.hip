@@ -196,8 +196,8 @@ struct OneTypeLJ
 //
 // With `staged` a block first copies the coefficients into its LDS as a square of num_types rows,
 // a pair's at type_i * num_types + type_j: a pair otherwise forms the row of its unordered types
-// and gathers four numbers from memory, a read as dear as that of its neighbor's position (two types:
-// 262,144 atoms 112 -> 90 us a step, 32,768 37.5 -> 33.9).
+// and gathers four numbers from memory, a read as dear as that of its neighbor's position (two
+// types: 262,144 atoms 112 -> 90 us a step, 32,768 37.5 -> 33.9).
 template <typename T>
 struct TypedLJ
 {
@@ -2200,7 +2200,7 @@ struct BrickShared
 {
     index_t run_first[kMaxBrickRuns];
     index_t run_rows[kMaxBrickRuns + 1];
-    double sums[16];
+    double sums[8 * 16];
 };
 
 // Bytes of a block's LDS past the halo.
@@ -2573,17 +2573,22 @@ __device__ __forceinline__ void force_body(const StepArgs<T>& a, const Launch la
             }
         }
     }
-    double* shared = sh->sums;
-    const double e = kEnergy ? block_sum(energy_sum, shared) : 0.0;
-    double v[6] = {0, 0, 0, 0, 0, 0};
+    // all of the block's sums behind one barrier: with one sum after another the seven of a step
+    // that needs the virial took 2 us of its 40 (10,007 atoms, fp64, NPT)
+    const int k = threadIdx.x;
     if (kVirial)
-        for (int k = 0; k < 6; ++k) v[k] = block_sum(w_sum[k], shared);
-    const double k_sum = kKick ? block_sum(kinetic, shared) : 0.0;
-    if (threadIdx.x == 0)
     {
-        out[0] = e;
-        for (int k = 0; k < 6; ++k) out[(1 + k) * column] = v[k];
-        out[7 * column] = k_sum;
+        double terms[8] = {kEnergy ? energy_sum : 0.0, w_sum[0], w_sum[1], w_sum[2], w_sum[3],
+                           w_sum[4], w_sum[5], kinetic};
+        const double sum = block_sums(terms, sh->sums);
+        if (k < 8) out[k * column] = sum;
+    }
+    else
+    {
+        // E or K alone, which thread 0 holds
+        double terms[1] = {kKick ? kinetic : energy_sum};
+        const double sum = block_sums(terms, sh->sums);
+        if (k < 8) out[(kKick ? (k + 7) % 8 : k) * column] = k == 0 ? sum : 0.0;
     }
 }
 
