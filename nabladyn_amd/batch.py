@@ -4,8 +4,8 @@
 LennardJones or Tabulated potential of this package — and evaluates energy, forces and virial of
 all of them with one binning pass, one scan and one force launch. ``schedule`` is "auto" (the
 autotuner times the four variants on this batch once and keeps the fastest), or one of
-("thread", 1), ("thread", 2), ("wave", 1), ("wave", 2): a lane or a wave per atom, and sub-bins
-at least the cutoff or half the cutoff wide.
+("thread", 1), ("thread", 2), ("wave", 1), ("wave", 2): a lane per atom or a wave per sub-bin, and
+sub-bins at least the cutoff or half the cutoff wide.
 
 ``plain_efw`` is the per-system path the batch is measured against: for each system, a
 ``NeighborList`` (zero skin) allocated on it and ``quantity.energy_force_virial`` — the
