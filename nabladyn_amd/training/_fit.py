@@ -172,14 +172,14 @@ def _chunks(frames: Tensor, size: int):
     yield from frames.split(size)
 
 
-def _pair_parts(model: Potential, prefix: str = ""):
-    """(parameter prefix, model) of each LJ or table in a model that is one or a sum of them,
-    None for any other (a subclass may compute otherwise)."""
+def _pair_parts(model: Potential):
+    """Each LJ or table in a model that is one or a sum of them, once per use; None for any other
+    (a subclass may compute otherwise)."""
     if type(model) in (LennardJones, Tabulated):
-        return [(prefix, model)]
+        return [model]
     if type(model) is not Sum:
         return None
-    parts = [_pair_parts(part, f"{prefix}parts.{k}.") for k, part in enumerate(model.parts)]
+    parts = [_pair_parts(part) for part in model.parts]
     return None if any(part is None for part in parts) else [p for part in parts for p in part]
 
 
@@ -200,9 +200,9 @@ def _kernel_gradient(model: Potential, parts, trained: dict[str, Tensor], prepar
     frames, rows, stacks and labels are read in place."""
     cutoffs = model._list_cutoffs
     rows, stacks = dict(zip(cutoffs, prepared.rows)), dict(zip(cutoffs, prepared.stacks))
-    natives = [part._native() for _, part in parts]
+    natives = [part._native() for part in parts]
     values = None
-    for (_, part), native in zip(parts, natives):
+    for part, native in zip(parts, natives):
         found = evaluate_frames_full(part, prepared.positions, prepared.cells,
                                      _loss._list_for(rows, part.cutoff), native, chunk)
         values = found if values is None else tuple(a + b for a, b in zip(values, found))
@@ -211,16 +211,20 @@ def _kernel_gradient(model: Potential, parts, trained: dict[str, Tensor], prepar
                                    [weights.get(name, 0.0) for name in _loss.CHANNELS],
                                    [channel_scales.get(name, 1.0) for name in _loss.CHANNELS],
                                    coefficient)
+    # by the tensor, not by a part's name for it: a tensor that several parts (or both rows of one)
+    # train is listed once among the trained, and takes the sum over its uses
+    names = {id(value): name for name, value in trained.items()}
     gradient = {}
-    for (prefix, part), native in zip(parts, natives):
-        names = [name for name, _ in part.named_parameters() if prefix + name in trained]
-        if not names:
+    for part, native in zip(parts, natives):
+        own = part._differentiable_parameters()
+        if not any(id(value) in names for value in own):
             continue
         g = parameter_vjp_frames(part, prepared.positions, prepared.cells,
                                  _loss._list_for(stacks, part.cutoff), *gradients, native, chunk)
-        split = part._split_parameter_gradient(g.to(model.dtype))
-        own = [name for name, _ in part.named_parameters()]
-        gradient.update((prefix + name, split[own.index(name)]) for name in names)
+        for value, piece in zip(own, part._split_parameter_gradient(g.to(model.dtype))):
+            name = names.get(id(value))
+            if name is not None:
+                gradient[name] = gradient[name] + piece if name in gradient else piece
     return gradient, terms[0], {name: terms[1 + k] for k, name in enumerate(_loss.CHANNELS)
                                 if name in prepared.labels}
 

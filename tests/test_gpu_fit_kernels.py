@@ -75,3 +75,63 @@ def test_kernel_gradient_equals_autograd(device, dtype, kind, n, channels):
         assert abs(float(loss) - float(loss0)) <= tight * abs(float(loss0))
         for name in terms:
             assert abs(float(terms[name]) - float(terms0[name])) <= tight * abs(float(terms0[name]))
+
+
+def _shared(kind, n, dtype, device, tied):
+    """A model in which one tensor trains under more than one name; untied, the same model with a
+    tensor of its own for each name."""
+    as_t = lambda v: torch.tensor(v, dtype=dtype, device=device)  # noqa: E731
+    zeros = torch.zeros(n, dtype=torch.int64, device=device)
+    lj = lambda sigma, epsilon, cutoff: potential.lennard_jones(  # noqa: E731
+        atom_types=zeros, sigma=as_t([sigma]), epsilon=as_t([epsilon]), cutoff=cutoff,
+        trainable=("sigma", "epsilon"))
+    if kind == "one tensor in one part":
+        only = lj(0.46, 0.46, 1.0)
+        if tied:
+            only.epsilon = only.sigma
+        return only
+    first, second = lj(0.46, 2.0, 1.0), lj(0.44, 2.0, 1.2)
+    again = first if tied else lj(0.46, 2.0, 1.0)
+    if kind == "one part twice":
+        return potential.sum(first, again)
+    if tied:
+        second.epsilon = first.epsilon
+    return potential.sum(first, potential.sum(second, again))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("kind", ["one part twice", "one tensor in one part",
+                                  "one tensor in two parts"])
+def test_shared_parameters_get_every_use(device, dtype, kind):
+    n, frames = 300, 4
+    rng = np.random.default_rng(5)
+    length = (n / 8.0) ** (1 / 3)
+    x = np.stack([workloads.lattice((7,) * 3, (length,) * 3, 0.04, rng, n=n)
+                  for _ in range(frames)])
+    as_np = lambda v: np.asarray(v).astype(np.float32 if dtype == torch.float32 else np.float64)  # noqa: E731
+    channels = ("energy", "forces", "virial")
+    data = training.Dataset(as_np(x), as_np(np.full((frames, 3), length)),
+                            energy=as_np(rng.normal(0, 50, frames)),
+                            forces=as_np(rng.normal(0, 30, (frames, n, 3))),
+                            virial=as_np(rng.normal(0, 80, (frames, 3, 3))))
+    model = _shared(kind, n, dtype, device, True)
+    twin = _shared(kind, n, dtype, device, False)
+    prepared = _fit._prepare(model, data, channels)
+    scales = training.scales(**prepared.labels)
+    weights = {name: 1.0 for name in channels}
+    own = dict(model.named_parameters())
+    chosen = torch.arange(frames)
+    g, loss, _ = _fit.batch_gradient(model, own, prepared, chosen, 3, weights, scales)
+    # through autograd, a tensor for each use, then the uses of one tensor added
+    copies = {name: p.detach().clone() for name, p in twin.named_parameters()}
+    uses, loss0, _ = _fit.batch_gradient(twin, copies, prepared, chosen, 3, weights, scales)
+    names = {id(p): name for name, p in own.items()}
+    g0 = {name: torch.zeros_like(p) for name, p in own.items()}
+    for name, p in model.named_parameters(remove_duplicate=False):
+        g0[names[id(p)]] += uses[name]
+    assert set(g) == set(g0)
+    # the parts' sums in fp64, each rounded and then added: an ulp a use beside the bounds above
+    loose = 1e-5 if dtype == torch.float32 else 1e-11
+    for name in g:
+        assert float((g[name] - g0[name]).abs().max()) <= loose * float(g0[name].abs().max()), name
+    assert abs(float(loss) - float(loss0)) <= loose * abs(float(loss0))
