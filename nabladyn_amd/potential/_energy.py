@@ -215,7 +215,10 @@ def frames_loss(predicted, labels, at: Tensor, weights, scales, coefficient: flo
     ``at`` (int64 [B]) names, and of every stored frame, a label None for a channel outside the
     loss; ``weights`` and ``scales`` are numbers, one per channel. Returns the gradients (None
     outside the loss) and [4]: the loss and the three unweighted terms."""
-    energy, forces, _ = predicted
+    # the kernel reads every array as its shape says
+    predicted = tuple(value.contiguous() for value in predicted)
+    labels = tuple(None if label is None else label.contiguous() for label in labels)
+    forces = predicted[1]
     frames, atoms, device = forces.shape[0], forces.shape[1], forces.device
     stored = next(v.shape[0] for v in labels if v is not None)
     gradients = tuple(None if label is None else torch.empty_like(value)

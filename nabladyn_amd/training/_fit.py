@@ -162,8 +162,10 @@ def _prepare(model: Potential, data: Dataset, channels: tuple[str, ...]) -> _Pre
     rows = None
     if model._fused:
         rows = tuple(_loss.frame_rows(stack, model.num_atoms) for stack in stacks)
-    return _Prepared(positions, cells, stacks,
-                     {name: moved(data.labels[name]) for name in channels}, rows)
+    # one layout for every label, whatever strides it was given with: the loss kernel reads them in
+    # place
+    labels = {name: moved(data.labels[name]).contiguous() for name in channels}
+    return _Prepared(positions, cells, stacks, labels, rows)
 
 
 def _chunks(frames: Tensor, size: int):

@@ -135,3 +135,36 @@ def test_shared_parameters_get_every_use(device, dtype, kind):
     for name in g:
         assert float((g[name] - g0[name]).abs().max()) <= loose * float(g0[name].abs().max()), name
     assert abs(float(loss) - float(loss0)) <= loose * abs(float(loss0))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+def test_labels_of_any_strides(device, dtype):
+    n, frames = 300, 5
+    rng = np.random.default_rng(6)
+    kind = np.float32 if dtype == torch.float32 else np.float64
+    length = (n / 8.0) ** (1 / 3)
+    x = np.stack([workloads.lattice((7,) * 3, (length,) * 3, 0.04, rng, n=n)
+                  for _ in range(frames)]).astype(kind)
+    cells = np.full((frames, 3), length, kind)
+    labels = {"energy": rng.normal(0, 50, frames).astype(kind),
+              "forces": rng.normal(0, 30, (frames, n, 3)).astype(kind),
+              "virial": rng.normal(0, 80, (frames, 3, 3)).astype(kind)}
+    strided = {"energy": torch.tensor(np.repeat(labels["energy"], 2))[::2],
+               "forces": torch.tensor(labels["forces"].transpose(0, 2, 1).copy()).transpose(1, 2),
+               "virial": np.asfortranarray(labels["virial"])}
+    model = _model("table", n, dtype, device)
+    own = dict(model.named_parameters())
+    out = []
+    for given in (labels, strided):
+        data = training.Dataset(x, cells, **given)
+        prepared = _fit._prepare(model, data, tuple(labels))
+        out.append(_fit.batch_gradient(model, own, prepared, torch.tensor([3, 0, 4]), 2,
+                                       {name: 1.0 for name in labels},
+                                       training.scales(**prepared.labels)))
+    # the same numbers in the same order; the scales and the VJP's sums (atomics) in another order
+    loose = 1e-5 if dtype == torch.float32 else 1e-11
+    for name in out[0][0]:
+        a, b = out[0][0][name], out[1][0][name]
+        assert float((a - b).abs().max()) <= loose * float(a.abs().max())
+    for name in labels:
+        assert abs(float(out[0][2][name]) - float(out[1][2][name])) <= loose * abs(float(out[0][2][name]))
