@@ -231,18 +231,35 @@ def _kernel_gradient(model: Potential, parts, trained: dict[str, Tensor], prepar
                                 if name in prepared.labels}
 
 
+def _frame_indices(frames: Tensor, stored: int):
+    """(the indices as the kernels take them, whether they may): int64 in [0, stored). Indices on
+    the host are checked here, a negative one counting from the end, and ``IndexError`` raised
+    for one outside the frames, which a kernel would pass over in silence. Any other choice (on
+    the device, a mask, ..) is left to indexing."""
+    if (frames.device.type != "cpu" or frames.ndim != 1
+            or frames.dtype not in (torch.int32, torch.int64)):
+        return frames, False
+    frames = frames.long()
+    outside = (frames < -stored) | (frames >= stored)
+    if bool(outside.any()):
+        raise IndexError(f"frames must lie in [{-stored}, {stored}), not "
+                         f"{int(frames[outside][0])}")
+    return torch.where(frames < 0, frames + stored, frames), True
+
+
 def batch_gradient(model: Potential, trained: dict[str, Tensor], prepared: _Prepared,
                    frames: Tensor, size: int, weights: dict[str, float],
                    channel_scales: dict[str, float]):
     """(gradient by name, loss, terms by name) of the mean loss over ``frames``, in chunks of
     ``size`` frames (``training/_fit.py:33-70``): each frame weighs 1/B, so the chunks' sums
-    equal the batch's."""
+    equal the batch's. Raises ``IndexError`` for a frame outside the prepared set."""
     channels = tuple(prepared.labels)
     leaves = {name: value.detach().requires_grad_(True) for name, value in trained.items()}
     device = prepared.positions.device
     gradient = {name: torch.zeros_like(value) for name, value in trained.items()}
     total_loss, total_terms = None, None
-    parts = _kernel_parts(model, trained, prepared)
+    frames, checked = _frame_indices(frames, prepared.positions.shape[0])
+    parts = _kernel_parts(model, trained, prepared) if checked else None
     for chunk in _chunks(frames, size):
         chunk = chunk.to(device)
         if parts is not None:

@@ -163,3 +163,27 @@ def test_frame_rows_list_every_pair_both_ways_in_stack_order():
         for s in range(per_frame):
             assert int(rows.slices[f, s + 1] - rows.slices[f, s]) == 64 * max(
                 widths[64 * s:64 * s + 64])
+
+
+def test_batch_gradient_refuses_frames_out_of_range():
+    """An index past the frames is an IndexError before anything is launched, a negative one counts
+    from the end, for a model's own parameters (which kernels alone differentiate) as for others."""
+    model = _lj()
+    trained = dict(model.named_parameters())
+    prepared = _fit._Prepared(torch.zeros(5, 8, 3, dtype=torch.float64), torch.ones(5, 3),
+                              (torch.zeros(5, 2, 4, dtype=torch.int32),), {},
+                              (None,))
+    for bad in ([0, 5], [-6], [1, 2, 7]):
+        with pytest.raises(IndexError, match="frames"):
+            _fit.batch_gradient(model, trained, prepared, torch.tensor(bad), 2, {}, {})
+    seen = []
+    original = _fit._kernel_gradient
+    _fit._kernel_gradient = lambda *a: (seen.append(a[4].tolist()),
+                                        ({}, torch.zeros(()), {}))[1]
+    try:
+        _fit.batch_gradient(model, trained, prepared, torch.tensor([-1, 0, -5]), 2, {}, {})
+        _fit.batch_gradient(model, trained, prepared, torch.tensor([4, 1], dtype=torch.int32), 2,
+                            {}, {})
+    finally:
+        _fit._kernel_gradient = original
+    assert seen == [[4, 0], [0], [4, 1]]
