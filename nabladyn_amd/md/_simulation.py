@@ -117,6 +117,10 @@ _BRICKS = ((4, 4, 8), (4, 2, 8), (2, 2, 8), (2, 2, 4), (2, 1, 4), (1, 1, 4), (1,
 # 28 / 34 us at 150 / 256 / 198 smaller ones; at 300 / 480 / 363 still smaller ones 29 / 29 / 35.
 _FILLING_BRICKS = 150
 
+# Bricks that all run at once, two blocks to a compute unit: up to here a halo's LDS, within the
+# half of a unit's that two blocks share, keeps no other block off the chip.
+_RESIDENT_BRICKS = 512
+
 
 def _brick_count(shape, dims) -> int:
     return math.prod(-(-d // b) for d, b in zip(dims, shape))
@@ -280,12 +284,17 @@ class _MDNeighbors:
 
     def size_halo(self, needed: int) -> None:
         """Room for halos of `needed` atoms with a margin (half the rows' multiplier's), up to
-        what LDS holds."""
+        what LDS holds. Where every brick is resident at once, all of that room (or every atom's):
+        the small bricks of a small system would otherwise run out of theirs as its atoms gather,
+        where a larger brick, whose halo may span the box, would not."""
         margin = self.halo_margin
         limit = halo_limit(self.dtype)
         # within the budget less the potential's share when the halo fits it (else as LDS allows)
         room = limit - self.reserve if needed <= limit - self.reserve else limit
-        capacity = min(max(1, math.ceil(margin * needed)), room)
+        wanted = math.ceil(margin * needed)
+        if self.bricks <= _RESIDENT_BRICKS:
+            wanted = max(wanted, self.buffers["counts"].numel())
+        capacity = min(max(1, wanted), room)
         self.buffers["halo_slots"] = torch.zeros(self.bricks * capacity, dtype=torch.int32,
                                                  device=self.buffers["counts"].device)
         self.native.halo_slots = _native.ptr(self.buffers["halo_slots"])
