@@ -240,11 +240,14 @@ def _frame_indices(frames: Tensor, stored: int):
             or frames.dtype not in (torch.int32, torch.int64)):
         return frames, False
     frames = frames.long()
-    outside = (frames < -stored) | (frames >= stored)
-    if bool(outside.any()):
-        raise IndexError(f"frames must lie in [{-stored}, {stored}), not "
-                         f"{int(frames[outside][0])}")
-    return torch.where(frames < 0, frames + stored, frames), True
+    # one pass over a handful of numbers: tensor operations would cost an update 25 us
+    values = frames.tolist()
+    low = min(values, default=0)
+    if low < -stored or max(values, default=0) >= stored:
+        raise IndexError(f"frames must lie in [{-stored}, {stored})")
+    if low < 0:
+        frames = torch.where(frames < 0, frames + stored, frames)
+    return frames, True
 
 
 def batch_gradient(model: Potential, trained: dict[str, Tensor], prepared: _Prepared,
