@@ -589,12 +589,17 @@ __device__ __forceinline__ bool refreshing(const StepArgs<T>& a)
 }
 
 // Whether a build kernel works on this step: the check asked for a build and no status bit is set
-// but the halo overflow of this very build. Its later phases stay in bounds past that (an atom
-// outside its halo's slots is listed as the sentinel) and report what else overflows.
+// but the overflows of this very build (the check asks for none while any bit is set, and clears
+// the request each step). A launch that may set one of them has other work in it, which must
+// reach every atom whichever block read the status first: the order beside the halo listing, the
+// unpack beside the fill. The later phases stay in bounds past an overflow (an atom outside its
+// halo's slots is listed as the sentinel, a row keeps its first `stride` entries) and report
+// what else overflows.
 template <typename T>
 __device__ __forceinline__ bool building(const StepArgs<T>& a)
 {
-    return a.rebuild[0] != 0 && (a.status[0] & ~kStatusHaloOverflow) == 0;
+    return a.rebuild[0] != 0 &&
+           (a.status[0] & ~(kStatusHaloOverflow | kStatusFullOverflow)) == 0;
 }
 
 // The block a kernel body runs as and the number of blocks of its system: the hardware's own in
@@ -1558,9 +1563,8 @@ inline std::size_t sort_bytes(std::int64_t bins)
 
 // The sort; with kWhole everything but the fill (the order with the halo listing, then the
 // frame home), its phases separated by the block's barriers instead of kernel boundaries. The
-// gate is read once per phase by one thread (a phase may set a status bit, and the phases after
-// it then do nothing, as the launches of a large build do); the bodies are those a large build
-// runs, so the list is the same bit for bit.
+// gate is read once per phase by one thread, so that the block goes on or stops as one; the bodies
+// are those a large build runs, so the list is the same bit for bit.
 template <typename T, bool kWhole>
 __global__ void __launch_bounds__(kListScanThreads) md_sort_kernel(StepArgs<T> a, int forced)
 {
@@ -2021,7 +2025,8 @@ __device__ __forceinline__ void md_fill_body(const StepArgs<T>& a, const Launch 
 
 // The unpack and the fill in one launch: neither reads what the other writes (the fill reads the
 // gather copy the order wrote, the halo lists and the sub-bin offsets; the unpack writes the
-// frame home), so the first `unpack_blocks` blocks unpack and the rest fill.
+// frame home), so the first `unpack_blocks` blocks unpack and the rest fill. The status bit that
+// the fill may set stops neither (building).
 template <typename T>
 __device__ __forceinline__ void md_unpack_fill_body(const StepArgs<T>& a, const Launch launch,
                                                     index_t unpack_blocks, T radius,

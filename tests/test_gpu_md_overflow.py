@@ -40,3 +40,20 @@ def test_a_box_that_halos_span_may_gather(device, dtype):
     got = sim.state().positions.cpu().numpy()
     np.testing.assert_allclose(got, expected, rtol=0, atol=2e-4)
     assert sim._neighbors._rebuild_count > 1
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("n", [1000, 1500, 5000])
+def test_a_row_overflow_moves_the_whole_frame(device, dtype, n):
+    """Rows that outgrow their entries stop a run with its error; the build that met them has still
+    put every atom home: each slot's mass and place are those of the atom it names. (1,000 atoms
+    take the build of one block and a fill, the others the launches that unpack beside the fill.)"""
+    length = 0.62 * np.ceil(n ** (1 / 3))
+    sim, x, v, masses = _gathering(device, dtype, n, length, 0.5, 100)
+    with pytest.raises(ValueError, match="a neighbor row needs"):
+        sim.run(100)
+    ids = sim._neighbors.buffers["ids"].cpu().numpy()
+    np.testing.assert_array_equal(np.sort(ids), np.arange(n))
+    np.testing.assert_array_equal(sim.slot_masses.cpu().numpy(), masses.cpu().numpy()[ids])
+    got = sim.positions.cpu().numpy()
+    np.testing.assert_allclose(got, (x + v * 0.4)[ids], rtol=0, atol=2e-4)
