@@ -531,9 +531,10 @@ int ndn_md_to_atom_order(int element_bytes, const void* in, const int32_t* ids, 
  * dims [3] of widths [3], each at least cutoff / span wide). Its potential is LJ (kinds = NDN_LJ,
  * lj_rows [4] = sigma^2, 4 eps, 24 eps, the energy at the cutoff) or a padded table row
  * (table_of >= 0 into tables [R, K + 2], table_start [R], table_spacing [R]). The rest
- * is scratch (bin_counts zero between calls; atom_terms [N, 7], partial sums of E and W in rows of
- * each system's own) and outputs: forces [N, 3], energy [S], virial [S, 3, 3]. Positions may lie outside their cells. No reference
- * counterpart: the reference evaluates one system per call. */
+ * is scratch (bin_counts zero between calls) and outputs: forces [N, 3], atom_terms [N, 7] (half
+ * of each atom's pair energies, then of its pair virials xx, yy, zz, xy, xz, yz), energy [S],
+ * virial [S, 3, 3]. Positions may lie outside their cells. No reference counterpart: the reference
+ * evaluates one system per call. */
 typedef struct ndn_batch {
     int64_t num_systems;
     int64_t num_atoms;

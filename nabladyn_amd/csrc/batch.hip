@@ -5,8 +5,8 @@
 // sort bins every atom of the batch, one scan covers every bin, and one force launch covers every
 // atom. The force launch builds no list: each atom's candidates come from the culled stencil of
 // its own system's sub-bins, and the pair terms are summed as they are found. Two schedules:
-//   - wave per sub-bin: its atoms' candidates 64 at a time across the lanes, read once for up to
-//     four atoms, reduced over the wave;
+//   - wave per sub-bin: its atoms' candidates 64 at a time across the lanes, read once for two
+//     atoms, reduced over the wave;
 //   - thread per atom: a lane per atom walking its own stencil.
 // and two sub-bin sizes (at least the cutoff, or half of it). A host-side autotuner times the
 // four on the batch and keeps the fastest.
@@ -61,7 +61,7 @@ struct BatchArgs
     std::uint8_t* scan_temp;
     // outputs
     T* forces;                     // [N, 3]
-    T* atom_terms;                 // [N, 7]: partial sums of E and W, a system's in its atoms' rows
+    T* atom_terms;                 // [N, 7]: half the pair energy and virial of each atom
     T* energy;                     // [S]
     T* virial;                     // [S, 9]
 };
@@ -349,14 +349,14 @@ struct WavePotential
     }
 };
 
-// Centers of a bin that a wave takes together, and the waves per SIMD its registers are held to
-// (fp32: 1.46 ms at 5 and 6 against 1.63 unbounded, for the 256 systems of 64 to 32,768 atoms;
-// three centers 1.50, two 1.53. fp64, 40 systems to 10,000 atoms: 257 us with three unbounded,
-// 267 with two, 273 bounded).
+// Centers of a bin that a wave takes together. Each keeps ten sums of its own (F, E and W, which
+// go out per atom), so more centers cost the waves that hide the gathers: the 256 systems of 64
+// to 32,768 atoms in fp32 take 1.46 ms with two centers at 7 or 8 waves per SIMD, 1.57 with three
+// at 6, 1.52 with four at 5; 40 systems to 10,000 atoms in fp64 237 us with two at 4, 246 with two
+// unbounded, 294 with three.
+constexpr int kWaveCenters = 2;
 template <typename T>
-constexpr int kWaveCenters = sizeof(T) == 4 ? 4 : 3;
-template <typename T>
-constexpr int kWaveOccupancy = sizeof(T) == 4 ? 5 : 1;
+constexpr int kWaveOccupancy = sizeof(T) == 4 ? 8 : 4;
 
 // How a candidate's vector is formed, uniform over a bin's centers.
 constexpr int kWavePlain = 0;    // the stencil lies inside the box
@@ -432,8 +432,7 @@ __device__ __forceinline__ void wave_range(const BatchArgs<T>& a, const SystemVi
     length = a.bin_offsets[base + last + 1] - lo;
 }
 
-// The sum over the wave by data-parallel moves (no LDS): rows of 16, then across the rows; the
-// total in lane 63.
+// A data-parallel move into kRows of the wave's rows of 16 lanes, zeros into the others.
 template <int kControl, int kRows>
 __device__ __forceinline__ float moved(float value)
 {
@@ -451,16 +450,35 @@ __device__ __forceinline__ double moved(double value)
     return __hiloint2double(hi, lo);
 }
 
-template <typename T>
-__device__ __forceinline__ T wave_total(T value)
+// a's halves added in the wave's lower half, b's in its upper: the upper half of a's lanes and
+// the lower half of b's change places, then one addition.
+__device__ __forceinline__ float folded(float a, float b)
 {
-    value += moved<0x111, 0xF>(value);  // row_shr:1
-    value += moved<0x112, 0xF>(value);  // row_shr:2
-    value += moved<0x114, 0xF>(value);  // row_shr:4
-    value += moved<0x118, 0xF>(value);  // row_shr:8
-    value += moved<0x142, 0xA>(value);  // row_bcast:15 into rows 1 and 3
-    value += moved<0x143, 0xC>(value);  // row_bcast:31 into rows 2 and 3
-    return value;
+    const auto both =
+        __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return __uint_as_float(both[0]) + __uint_as_float(both[1]);
+}
+
+__device__ __forceinline__ double folded(double a, double b)
+{
+    const auto lo =
+        __builtin_amdgcn_permlane32_swap(__double2loint(a), __double2loint(b), false, false);
+    const auto hi =
+        __builtin_amdgcn_permlane32_swap(__double2hiint(a), __double2hiint(b), false, false);
+    return __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
+}
+
+// Two sums over the wave at once, a's in lane 31 and b's in lane 63, without LDS.
+template <typename T>
+__device__ __forceinline__ T two_sums(T a, T b)
+{
+    T sum = folded(a, b);
+    sum += moved<0x111, 0xF>(sum);  // row_shr:1
+    sum += moved<0x112, 0xF>(sum);  // row_shr:2
+    sum += moved<0x114, 0xF>(sum);  // row_shr:4
+    sum += moved<0x118, 0xF>(sum);  // row_shr:8
+    sum += moved<0x142, 0xA>(sum);  // row_bcast:15 into rows 1 and 3
+    return sum;
 }
 
 // A group of a bin's centers (slots first .. first + live - 1) against their candidates, 64 a
@@ -471,7 +489,7 @@ __device__ __forceinline__ void wave_centers(const BatchArgs<T>& a, const System
                                              index_t first, int live, T reach)
 {
     using V4 = typename std::conditional<sizeof(T) == 4, float4, double4>::type;
-    constexpr int kCenters = kWaveCenters<T>;
+    constexpr int kCenters = kWaveCenters;
     const int lane = lane_id();
     const V4* sorted = reinterpret_cast<const V4*>(a.sorted4);
     const V4 own = sorted[first + (lane < live ? lane : 0)];
@@ -497,11 +515,13 @@ __device__ __forceinline__ void wave_centers(const BatchArgs<T>& a, const System
     const index_t start = inclusive - length;
     const index_t to_slot = lo - start;
     const index_t total = read_lane(inclusive, kWave - 1);
-    T fx[kCenters], fy[kCenters], fz[kCenters];
+    // each center's F, E and W
+    constexpr int kSums = 10;
+    T sums[kSums][kCenters];
 #pragma unroll
-    for (int g = 0; g < kCenters; ++g) fx[g] = fy[g] = fz[g] = T(0);
-    T e = 0;
-    T w[6] = {0, 0, 0, 0, 0, 0};
+    for (int k = 0; k < kSums; ++k)
+#pragma unroll
+        for (int g = 0; g < kCenters; ++g) sums[k][g] = T(0);
     for (index_t chunk = 0; chunk < total; chunk += kWave)
     {
         const index_t t = chunk + lane;
@@ -552,51 +572,38 @@ __device__ __forceinline__ void wave_centers(const BatchArgs<T>& a, const System
                 T u, fs;
                 pot.eval(r2, u, fs);
                 const T gx = fs * dx, gy = fs * dy, gz = fs * dz;
-                e += u;
-                fx[g] += gx;
-                fy[g] += gy;
-                fz[g] += gz;
-                w[0] += dx * gx;
-                w[1] += dy * gy;
-                w[2] += dz * gz;
-                w[3] += dx * gy;
-                w[4] += dx * gz;
-                w[5] += dy * gz;
+                sums[0][g] += gx;
+                sums[1][g] += gy;
+                sums[2][g] += gz;
+                sums[3][g] += u;
+                sums[4][g] += dx * gx;
+                sums[5][g] += dy * gy;
+                sums[6][g] += dz * gz;
+                sums[7][g] += dx * gy;
+                sums[8][g] += dx * gz;
+                sums[9][g] += dy * gz;
             }
         }
     }
+    T out[kSums];
 #pragma unroll
-    for (int g = 0; g < kCenters; ++g)
+    for (int k = 0; k < kSums; ++k) out[k] = two_sums(sums[k][0], sums[k][1]);
+    // lane 31 holds the first center's, lane 63 the second's
+    const int g = lane / 32;
+    if (lane % 32 == 31 && g < live)
     {
-        if (g >= live) break;
-        const T sx = wave_total(fx[g]), sy = wave_total(fy[g]), sz = wave_total(fz[g]);
-        if (lane == kWave - 1)
-        {
-            T* f = a.forces + 3LL * a.order[first + g];
-            f[0] = sx;
-            f[1] = sy;
-            f[2] = sz;
-        }
+        const index_t atom = a.order[first + g];
+        T* f = a.forces + 3LL * atom;
+        T* terms = a.atom_terms + 7LL * atom;
+        for (int k = 0; k < 3; ++k) f[k] = out[k];
+        for (int k = 0; k < 7; ++k) terms[k] = T(0.5) * out[3 + k];
     }
-    // the group's E and W in its first slot's terms, zeros in the others'
-    const T se = wave_total(e);
-    T sw[6];
-    for (int k = 0; k < 6; ++k) sw[k] = wave_total(w[k]);
-    if (lane == kWave - 1)
-    {
-        T* terms = a.atom_terms + 7LL * first;
-        terms[0] = T(0.5) * se;
-        for (int k = 0; k < 6; ++k) terms[1 + k] = T(0.5) * sw[k];
-    }
-    if (lane >= 7 && lane < 7 * live) a.atom_terms[7LL * first + lane] = T(0);
 }
 
-// Wave per sub-bin. Its atoms share their stencil: the ranges, their prefix sums, each candidate's
-// place and image and the reductions of E and W are found once for up to four of them, where a
-// wave per atom spent most of its instructions on these. Bound by the issue of vector
-// instructions (about a third of the lanes of a chunk of candidates hold a pair). The 256 systems
-// (0.9 million atoms, half LJ, half tables): 2.08 -> 1.45 ms an evaluation at sub-bins of half
-// the cutoff, 3.68 -> 2.10 at sub-bins of the cutoff.
+// Wave per sub-bin. Its atoms share their stencil: the ranges, their prefix sums and each
+// candidate's place and image are found once for two of them, where a wave per atom spent most of
+// its instructions on these. The 256 systems (0.9 million atoms, half LJ, half tables): 1.97 ->
+// 1.46 ms an evaluation at sub-bins of half the cutoff, 3.68 -> 2.36 at sub-bins of the cutoff.
 template <typename T>
 __global__ void __launch_bounds__(kBlock, kWaveOccupancy<T>)
 batch_wave_kernel(BatchArgs<T> a, T cull_factor)
@@ -624,7 +631,7 @@ batch_wave_kernel(BatchArgs<T> a, T cull_factor)
     const bool inside = home[0] >= a.span && home[0] + a.span < v.nx && home[1] >= a.span &&
                         home[1] + a.span < v.ny && home[2] >= a.span && home[2] + a.span < v.nz;
     const T reach = v.cutoff * cull_factor;
-    constexpr int kCenters = kWaveCenters<T>;
+    constexpr int kCenters = kWaveCenters;
     for (index_t first = begin; first < end; first += kCenters)
     {
         const int live = end - first < kCenters ? end - first : kCenters;

@@ -71,3 +71,37 @@ def test_wave_per_bin_at_its_edges(device, dtype, span):
         assert rel(f.cpu(), f0) <= bar, k
         assert rel(virial[k].cpu(), w0) <= bar, k
         assert abs(float(energy[k]) - e0) <= bar * max(1.0, abs(e0)), k
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("schedule", batch.SCHEDULES)
+def test_terms_of_each_atom(device, dtype, schedule):
+    """``atom_terms``: half of each atom's pair energies and virials, whatever the schedule. Closed
+    forms in fp64 at the frames' own positions; bars as above, of each system's largest term."""
+    rng = np.random.default_rng(23)
+    sigma, epsilon, cutoff = 0.22, 0.996, 1.0
+    as_t = lambda v: torch.tensor(np.asarray(v), dtype=dtype, device=device)  # noqa: E731
+    systems = []
+    for x, cell in _frames(rng):
+        types = torch.zeros(len(x), dtype=torch.int64, device=device)
+        systems.append((as_t(x), as_t(cell), potential.lennard_jones(
+            atom_types=types, sigma=as_t([sigma]), epsilon=as_t([epsilon]), cutoff=cutoff)))
+    b = batch.Batch(systems, schedule=schedule)
+    b.evaluate()
+    bar = 1e-5 if dtype == torch.float32 else 1e-12
+    shift = 4 * epsilon * ((sigma / cutoff) ** 12 - (sigma / cutoff) ** 6)
+    for terms, (x, cell, _) in zip(b.split(b.atom_terms), systems):
+        x, cell = x.double().cpu().numpy(), cell.double().cpu().numpy()
+        d = x[:, None] - x[None]
+        d -= cell * np.round(d / cell)
+        r2 = (d ** 2).sum(-1)
+        np.fill_diagonal(r2, np.inf)
+        near = r2 < cutoff ** 2
+        s6 = np.where(near, sigma ** 6 / r2 ** 3, 0.0)
+        energy = np.where(near, 4 * epsilon * (s6 ** 2 - s6) - shift, 0.0)
+        scale = 24 * epsilon * (2 * s6 ** 2 - s6) / r2
+        expected = 0.5 * np.stack([energy.sum(1)] + [
+            (scale * d[..., p] * d[..., q]).sum(1)
+            for p, q in ((0, 0), (1, 1), (2, 2), (0, 1), (0, 2), (1, 2))], axis=1)
+        got = terms.double().cpu().numpy()
+        assert np.abs(got - expected).max() <= bar * max(np.abs(expected).max(), 1e-300)
