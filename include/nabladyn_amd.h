@@ -578,7 +578,8 @@ typedef struct ndn_batch {
 int64_t ndn_batch_scan_bytes(int64_t total_bins);
 
 /* E, F, W of every system of the batch: bin, sort, and one force launch over all atoms with no
- * stored list; schedule 0 = a lane per atom, 1 = a wave per sub-bin. */
+ * stored list; schedule 0 = a lane per atom, 1 = a wave per sub-bin or, where
+ * these are many or crowded, per pair of its atoms. */
 int ndn_batch_efw(int dtype, const ndn_batch* batch, int schedule, ndn_stream_t stream);
 
 /* Workspace bytes of ndn_batch_table_vjp. */

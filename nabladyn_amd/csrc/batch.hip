@@ -351,12 +351,12 @@ struct WavePotential
 
 // Centers of a bin that a wave takes together. Each keeps ten sums of its own (F, E and W, which
 // go out per atom), so more centers cost the waves that hide the gathers: the 256 systems of 64
-// to 32,768 atoms in fp32 take 1.46 ms with two centers at 7 or 8 waves per SIMD, 1.57 with three
-// at 6, 1.52 with four at 5; 40 systems to 10,000 atoms in fp64 237 us with two at 4, 246 with two
-// unbounded, 294 with three.
+// to 32,768 atoms in fp32 take 1.46 ms with two centers at 7 waves per SIMD (1.53 at 6), 1.57 with
+// three at 6, 1.52 with four at 5; 40 systems to 10,000 atoms in fp64 237 us with two at 4, 246
+// with two unbounded, 294 with three.
 constexpr int kWaveCenters = 2;
 template <typename T>
-constexpr int kWaveOccupancy = sizeof(T) == 4 ? 8 : 4;
+constexpr int kWaveOccupancy = sizeof(T) == 4 ? 7 : 4;
 
 // How a candidate's vector is formed, uniform over a bin's centers.
 constexpr int kWavePlain = 0;    // the stencil lies inside the box
@@ -604,18 +604,50 @@ __device__ __forceinline__ void wave_centers(const BatchArgs<T>& a, const System
 // candidate's place and image are found once for two of them, where a wave per atom spent most of
 // its instructions on these. The 256 systems (0.9 million atoms, half LJ, half tables): 1.97 ->
 // 1.46 ms an evaluation at sub-bins of half the cutoff, 3.68 -> 2.36 at sub-bins of the cutoff.
+//
+// A bin's atoms are taken in groups from its first, whatever else the batch holds, so that a system
+// gets the same bits alone and beside others. The groups that begin within a bin's first `share`
+// slots are its own wave's; those past them go to waves by slot, after the bins': wave `bins` + x
+// takes the groups beginning in [share x, share x + share) that lie as far into their bin, so that
+// a clump of atoms is spread over the chip. With `bins` 0 there is no wave per sub-bin: wave s
+// takes the group that begins at slot s, if one does.
 template <typename T>
 __global__ void __launch_bounds__(kBlock, kWaveOccupancy<T>)
-batch_wave_kernel(BatchArgs<T> a, T cull_factor)
+batch_wave_kernel(BatchArgs<T> a, T cull_factor, std::int64_t bins, index_t share)
 {
-    const std::int64_t bin = static_cast<std::int64_t>(blockIdx.x) * (kBlock / kWave) +
-                             __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    if (bin >= a.total_bins) return;
+    constexpr int kCenters = kWaveCenters;
+    const std::int64_t wave = static_cast<std::int64_t>(blockIdx.x) * (kBlock / kWave) +
+                              __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const bool by_slot = wave >= bins;
+    std::int64_t bin = wave;
+    index_t slot = 0, s = 0;
+    if (by_slot)
+    {
+        const std::int64_t at = (wave - bins) * share;
+        if (at >= a.num_atoms) return;
+        slot = static_cast<index_t>(at);
+        const index_t atom = __builtin_amdgcn_readfirstlane(a.order[slot]);
+        bin = __builtin_amdgcn_readfirstlane(a.bin_of[atom]);
+        s = __builtin_amdgcn_readfirstlane(a.system_of[atom]);
+    }
     const index_t begin = __builtin_amdgcn_readfirstlane(a.bin_offsets[bin]);
     const index_t end = __builtin_amdgcn_readfirstlane(a.bin_offsets[bin + 1]);
     if (begin == end) return;
-    const index_t s = __builtin_amdgcn_readfirstlane(a.system_of[a.order[begin]]);
+    if (!by_slot) s = __builtin_amdgcn_readfirstlane(a.system_of[a.order[begin]]);
+    // before the groups are known, so that its reads wait beside theirs
     const SystemView<T> v = system_view(a, s);
+    // the groups that begin in [from, past); differences, as a sum past the last slot could leave
+    // 32 bits
+    const index_t own = bins == 0 ? begin : (end - begin < share ? end : begin + share);
+    index_t from = begin, past = own;
+    if (by_slot)
+    {
+        from = slot > own ? slot : own;
+        past = end - slot < share ? end : slot + share;
+        from += (from - begin) % kCenters;
+        static_assert(kCenters == 2, "the next group's begin");
+    }
+    if (from >= past) return;
     WavePotential<T> pot;
     pot.kind = __builtin_amdgcn_readfirstlane(v.kind);
     pot.knots = a.knots;
@@ -631,8 +663,7 @@ batch_wave_kernel(BatchArgs<T> a, T cull_factor)
     const bool inside = home[0] >= a.span && home[0] + a.span < v.nx && home[1] >= a.span &&
                         home[1] + a.span < v.ny && home[2] >= a.span && home[2] + a.span < v.nz;
     const T reach = v.cutoff * cull_factor;
-    constexpr int kCenters = kWaveCenters;
-    for (index_t first = begin; first < end; first += kCenters)
+    for (index_t first = from; first < past; first += kCenters)
     {
         const int live = end - first < kCenters ? end - first : kCenters;
         if (image)
@@ -903,6 +934,28 @@ __global__ void __launch_bounds__(kReduceThreads) batch_reduce_kernel(BatchArgs<
     }
 }
 
+// How the wave schedule splits a batch.
+struct WaveShares
+{
+    std::int64_t waves, bins;
+    index_t share;
+};
+
+// Batches with fewer atoms than sub-bins go by slot: a wave per sub-bin finds most of them empty (40
+// systems of 500 atoms in boxes of 20 nm, sub-bins of half the cutoff: LJ 257 -> 65 us an
+// evaluation, tables 180 -> 61). With fewer sub-bins than waves fill the chip twice over (256
+// units of 4 SIMDs of 7), every group is a wave's own (20 systems of 4,000 atoms at 100 a nm3: LJ
+// 310 -> 233, tables 957 -> 459). Above, a wave takes four groups, which costs the uniform frames
+// nothing (the 256 systems 1,468 us with four or 32) and spreads a clump (100 systems of 9,000
+// atoms beside one whose half lies in a clump: LJ 6,125 us with a wave per sub-bin, 2,386 with 32
+// groups a wave, 1,093 with four).
+inline WaveShares wave_shares(std::int64_t atoms, std::int64_t bins)
+{
+    if (atoms < bins) return {atoms, 0, 1};
+    const index_t share = bins < 16384 ? kWaveCenters : 4 * kWaveCenters;
+    return {bins + (atoms + share - 1) / share, bins, share};
+}
+
 template <typename T>
 BatchArgs<T> batch_args(const ndn_batch& b);
 
@@ -925,8 +978,11 @@ int batch_impl(const ndn_batch& b, int schedule, hipStream_t stream)
     if (schedule == 0)
         batch_thread_kernel<T><<<blocks_for(n), kBlock, 0, stream>>>(a, cull_factor);
     else
-        batch_wave_kernel<T><<<blocks_for(a.total_bins, kBlock / kWave), kBlock, 0, stream>>>(
-            a, cull_factor);
+    {
+        const WaveShares w = wave_shares(n, a.total_bins);
+        batch_wave_kernel<T><<<blocks_for(w.waves, kBlock / kWave), kBlock, 0, stream>>>(
+            a, cull_factor, w.bins, w.share);
+    }
     NDN_LAUNCHED("batch_forces");
     batch_reduce_kernel<T><<<static_cast<unsigned>(b.num_systems), kReduceThreads, 0, stream>>>(a);
     NDN_LAUNCHED("batch_reduce");

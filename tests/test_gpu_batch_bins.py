@@ -105,3 +105,52 @@ def test_terms_of_each_atom(device, dtype, schedule):
             for p, q in ((0, 0), (1, 1), (2, 2), (0, 1), (0, 2), (1, 2))], axis=1)
         got = terms.double().cpu().numpy()
         assert np.abs(got - expected).max() <= bar * max(np.abs(expected).max(), 1e-300)
+
+
+def _crowded(rng):
+    """Clumps whose sub-bins hold hundreds of atoms, beside sparse frames: (few systems, so few
+    sub-bins and a pair of atoms a wave), (over 16,384 sub-bins, not more than atoms), (more
+    sub-bins than atoms, so waves by slot)."""
+    def frame(n, clump, sigma, length):
+        x = np.concatenate([rng.normal(length / 2, sigma, (clump, 3)),
+                            rng.uniform(0, length, (n - clump, 3))])
+        return x, (length,) * 3
+    few = [frame(1500, 900, 0.3, 5.0), frame(700, 0, 1, 2.6), frame(3, 0, 1, 2.6)]
+    return {"few bins": few,
+            "many bins": few + [frame(9000, 2000, 0.3, 8.0) for _ in range(8)],
+            "more bins than atoms": [frame(1500, 1200, 0.3, 9.0), frame(40, 0, 1, 12.0)]}
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("kind", ["few bins", "many bins", "more bins than atoms"])
+def test_clumps_spread_over_waves(device, dtype, kind):
+    """Every atom is some wave's center once: the wave schedule against the thread schedule, which
+    walks a stencil per atom. A table reaching zero distance keeps every term finite where atoms
+    overlap. Both add the same pair terms in the dtype, in other orders: an atom of P pairs to P
+    2^-24 of its summed |terms| (2^-53 in fp64), and P is below 2,000."""
+    systems = []
+    as_t = lambda v: torch.tensor(np.asarray(v), dtype=dtype, device=device)  # noqa: E731
+    knots = 121
+    table = 5.0 * (1.0 - np.arange(knots) / (knots - 1.0)) ** 2
+    for x, cell in _crowded(np.random.default_rng(31))[kind]:
+        systems.append((as_t(x), as_t(cell), potential.tabulated(
+            atom_types=torch.zeros(len(x), dtype=torch.int64, device=device),
+            table=as_t(table[None]), start=as_t([0.0]), cutoff=1.2)))
+    atoms = sum(len(x) for x, _, _ in systems)
+    for span in (1, 2):
+        a, b = (batch.Batch(systems, schedule=(way, span)) for way in ("thread", "wave"))
+        ea, fa, va = (v.double().cpu() for v in a.evaluate())
+        eb, fb, vb = (v.double().cpu() for v in b.evaluate())
+        if span == 2:
+            bins = sum(int(v) for v in b._layout(2).keep["dims"].prod(dim=1))
+            assert {"few bins": bins <= atoms and bins < 16384,
+                    "many bins": 16384 <= bins <= atoms,
+                    "more bins than atoms": bins > atoms}[kind]
+        bar = 2000 * (2.0 ** -24 if dtype == torch.float32 else 2.0 ** -53)
+        # |force| of a pair is at most the table's steepest slope, 2 * 5 / 1.2
+        pairs = 2000
+        assert float((fa - fb).abs().max()) <= bar * pairs * 2 * 5.0 / 1.2
+        ta, tb = a.atom_terms.double().cpu(), b.atom_terms.double().cpu()
+        assert float((ta - tb).abs().max()) <= bar * float(ta.abs().max())
+        assert float((ea - eb).abs().max()) <= bar * float(ea.abs().max())
+        assert float((va - vb).abs().max()) <= bar * float(va.abs().max())
