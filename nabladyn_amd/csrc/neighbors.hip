@@ -397,6 +397,9 @@ struct SearchArgs
     const index_t* dims;
     const T* cell;
     T radius_squared;
+    const index_t* atom_bin;
+    index_t num_atoms;
+    index_t share;                // slots of a bin to a block
     std::int64_t bin_slots;
     // count
     index_t* pair_counts;
@@ -470,14 +473,29 @@ __device__ __forceinline__ SearchRange search_range(const SearchArgs<T>& a, inde
 constexpr int kSearchWaves = 4;
 constexpr int kSearchPerLane = 4;
 
+// Slots of a bin that one block takes as centers, at most: 64 up to 524,288 atoms, and 128 above,
+// as most of the blocks by slot (search_pairs_kernel) have nothing to do in most frames (2,097,152
+// atoms: an idle update 70 us without them, 82 with 64 slots, 76 with 128). At 100 atoms a bin
+// (100,000 atoms, full list) a rebuild takes 668 us with 64, 688 with 128; at 125 (8,000 atoms)
+// 325 and 535.
+constexpr int kSearchShare = 128;
+constexpr std::int64_t kSmallShares = 524288;
+inline index_t search_share(std::int64_t atoms)
+{
+    return atoms <= kSmallShares ? kSearchShare / 2 : kSearchShare;
+}
+
 template <typename T>
 struct SearchTile
 {
     static constexpr int kRaw = kSearchWaves * kWave * kSearchPerLane;  // candidates read per tile
     T x[kRaw], y[kRaw], z[kRaw];
-    index_t slot[kRaw], id[kRaw], shift[kRaw];
+    index_t slot[kRaw], id[kRaw];
+    std::uint8_t shift[kRaw];
     index_t start[kSearchRanges], to_slot[kSearchRanges], range_shift[kSearchRanges];
     index_t kept[kSearchWaves * kSearchPerLane];
+    // the centers' running places between one tile and the next
+    index_t half[kSearchShare], row[kSearchShare];
     T box[6];
 };
 
@@ -563,7 +581,7 @@ __device__ __forceinline__ index_t stage_candidates(const SearchArgs<T>& a,
             tile.z[at] = pz[u];
             tile.slot[at] = slot[u];
             if (kFill) tile.id[at] = id[u];
-            if (kMode == kSearchShifted) tile.shift[at] = shift[u];
+            if (kMode == kSearchShifted) tile.shift[at] = static_cast<std::uint8_t>(shift[u]);
         }
     __syncthreads();
     static_assert(Tile::kRaw == kThreads * kSearchPerLane, "one candidate per lane and turn");
@@ -671,6 +689,9 @@ __device__ __forceinline__ void search_tile(const SearchArgs<T>& a,
     }
 }
 
+// The centers [begin, end), at most kSearchShare slots of a bin, against its candidates: a tile at a
+// time, and for each tile kSearchWaves groups of centers a turn. Most bins' candidates are one
+// tile; past it the centers' places wait in LDS for the next, so that every tile is read once.
 template <typename T, bool kFull, bool kFill, int kMode>
 __device__ __forceinline__ void search_bin(const SearchArgs<T>& a, SearchTile<T>& tile,
                                            index_t begin, index_t end, index_t total)
@@ -680,26 +701,38 @@ __device__ __forceinline__ void search_bin(const SearchArgs<T>& a, SearchTile<T>
     const int lane = lane_id();
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const T lx = a.cell[0], ly = a.cell[1], lz = a.cell[2];
-    // a candidate this far from the box of the bin's atoms pairs with none of them, whatever the
+    // a candidate this far from the box of the centers pairs with none of them, whatever the
     // rounding of its image
     const T radius = sqrt(a.radius_squared);
     const T longest = fmax(lx, fmax(ly, lz));
     const T reach = radius * T(1.001) + T(16) * std::numeric_limits<T>::epsilon() * longest;
     const T reach_squared = reach * reach;
-    index_t staged = -1, count = 0;
-    for (index_t round = begin; round < end; round += kSearchWaves * kCenters)
+    for (index_t base = 0; base == 0 || base < total; base += Tile::kRaw)
     {
-        const index_t first = round + wave * kCenters;
-        const int live = first >= end ? 0 : (end - first < kCenters ? end - first : kCenters);
-        const index_t mine = first + (lane < live ? lane : 0);
-        SearchGroup<T> c;
-        if (live > 0)
+        if (base > 0) __syncthreads();
+        const index_t count =
+            stage_candidates<T, kFill, kMode>(a, tile, base, total, lx, ly, lz, reach_squared);
+        const bool last = total - base <= Tile::kRaw;
+        for (index_t round = begin; round < end; round += kSearchWaves * kCenters)
         {
+            const index_t first = round + wave * kCenters;
+            const int live = first >= end ? 0 : (end - first < kCenters ? end - first : kCenters);
+            if (live == 0) continue;
+            const index_t mine = first + (lane < live ? lane : 0);
             const T mx = a.sp[3LL * mine], my = a.sp[3LL * mine + 1], mz = a.sp[3LL * mine + 2];
             const index_t id = kFill ? a.sorted_ids[mine] : 0;
-            const index_t column = kFill ? a.pair_offsets[mine] : 0;
-            const index_t entry =
-                kFill && kFull ? a.full_slices[mine / kWave] + mine % kWave : 0;
+            index_t half, row;
+            if (base > 0)
+            {
+                half = tile.half[mine - begin];
+                row = tile.row[mine - begin];
+            }
+            else
+            {
+                half = kFill ? a.pair_offsets[mine] : 0;
+                row = kFill && kFull ? a.full_slices[mine / kWave] + mine % kWave : 0;
+            }
+            SearchGroup<T> c;
 #pragma unroll
             for (int g = 0; g < kCenters; ++g)
             {
@@ -707,63 +740,82 @@ __device__ __forceinline__ void search_bin(const SearchArgs<T>& a, SearchTile<T>
                 c.y[g] = read_lane(my, g);
                 c.z[g] = read_lane(mz, g);
                 c.id[g] = read_lane(id, g);
-                c.half[g] = read_lane(column, g);
-                c.row[g] = read_lane(entry, g);
+                c.half[g] = read_lane(half, g);
+                c.row[g] = read_lane(row, g);
             }
-        }
-        for (index_t base = 0; base < total; base += Tile::kRaw)
-        {
-            if (staged != base)
-            {
-                if (staged >= 0) __syncthreads();
-                count = stage_candidates<T, kFill, kMode>(a, tile, base, total, lx, ly, lz,
-                                                                  reach_squared);
-                staged = base;
-            }
-            if (live > 0)
-                search_tile<T, kFull, kFill, kMode>(a, tile, count, first, live, lx, ly,
-                                                            lz, c);
-        }
-        if (!kFill)
-        {
-            index_t half = 0, full = 0;
+            search_tile<T, kFull, kFill, kMode>(a, tile, count, first, live, lx, ly, lz, c);
+            if (kFill && last) continue;
 #pragma unroll
             for (int g = 0; g < kCenters; ++g)
             {
                 half = lane == g ? c.half[g] : half;
-                full = lane == g ? c.row[g] : full;
+                row = lane == g ? c.row[g] : row;
             }
             if (lane < live)
             {
-                a.pair_counts[mine] = half;
-                if (kFull)
+                if (last)
                 {
-                    a.full_counts[mine] = full;
-                    atomicMax(a.full_slices + mine / kWave, full * kWave);
+                    a.pair_counts[mine] = half;
+                    if (kFull)
+                    {
+                        a.full_counts[mine] = row;
+                        atomicMax(a.full_slices + mine / kWave, row * kWave);
+                    }
+                }
+                else
+                {
+                    // read by the same lane
+                    tile.half[mine - begin] = half;
+                    tile.row[mine - begin] = row;
                 }
             }
         }
     }
 }
 
-// A block per bin. The candidates of a bin are the same for all its atoms: the block reads them
-// once into LDS, leaving out those out of reach of the box of the bin's atoms (a quarter of the
-// 27 bins' atoms at 28 atoms a bin), and each wave tests its centers against them. Bound by the
-// issue of vector and scalar instructions (about 11 of each per center and 64 candidates). A
-// lane per center, each writing columns of its own, wrote the lists 4 bytes to a line. A rebuild
-// at 2,097,152 atoms, radius 1.1 nm, full list: 6.9 -> 2.2 ms (the fill 5.8 -> 1.36, the count
-// 1.05 -> 0.72); a fill of 4,096 atoms, whose 64 waves left the chip idle, 140 -> 13 us.
+// A block per bin, or per share of a crowded one. The candidates of a bin are the same for all its
+// atoms: the block reads them into LDS, leaving out those out of reach of the box of its centers
+// (a quarter of the 27 bins' atoms at 28 atoms a bin), and each wave tests its centers against
+// them. Bound by the issue of vector and scalar instructions (about 11 of each per center and 64
+// candidates). A lane per center, each writing columns of its own, wrote the lists 4 bytes to a
+// line. A rebuild at 2,097,152 atoms, radius 1.1 nm, full list: 6.9 -> 2.1 ms (the fill 5.8 ->
+// 1.36, the count 1.05 -> 0.72); a fill of 4,096 atoms, whose 64 waves left the chip idle, 140 ->
+// 13 us.
+//
+// A bin of more atoms than a share leaves the rest to blocks by slot, past those of the bins:
+// block `bins` + x takes those of the slots [share x, share x + share) that lie as far into their
+// bin. 100,000 atoms, half of them in a clump of 1 nm: 27 ms a rebuild with a lane per center, 125
+// with a block per bin whatever it holds, 13 so; at 291 atoms a bin 5.2, 3.5 and 2.2.
 template <typename T, bool kFull, bool kFill>
 __global__ void __launch_bounds__(kSearchWaves * kWave) search_pairs_kernel(SearchArgs<T> a)
 {
     __shared__ SearchTile<T> tile;
     if (!rebuilding(a.rebuild, a.status)) return;
-    const std::int64_t bin = blockIdx.x;
     const index_t nx = a.dims[0], ny = a.dims[1], nz = a.dims[2];
-    if (bin >= static_cast<std::int64_t>(nx) * ny * nz || bin >= a.bin_slots - 1) return;
-    const index_t begin = __builtin_amdgcn_readfirstlane(a.bin_offsets[bin]);
-    const index_t end = __builtin_amdgcn_readfirstlane(a.bin_offsets[bin + 1]);
-    if (begin == end) return;
+    const std::int64_t bins = a.bin_slots - 1;
+    std::int64_t bin = blockIdx.x;
+    index_t slot = 0;
+    if (bin >= bins)
+    {
+        // a block by slot
+        const std::int64_t at = (bin - bins) * a.share;
+        if (at >= a.num_atoms) return;
+        slot = static_cast<index_t>(at);
+        bin = __builtin_amdgcn_readfirstlane(a.atom_bin[a.sorted_ids[slot]]);
+    }
+    if (bin >= static_cast<std::int64_t>(nx) * ny * nz || bin >= bins) return;
+    index_t begin = __builtin_amdgcn_readfirstlane(a.bin_offsets[bin]);
+    index_t end = __builtin_amdgcn_readfirstlane(a.bin_offsets[bin + 1]);
+    // the bin's own block ends here (differences: a sum past the last slot could leave 32 bits)
+    const index_t own = end - begin < a.share ? end : begin + a.share;
+    if (blockIdx.x < bins)
+        end = own;
+    else
+    {
+        begin = slot > own ? slot : own;
+        end = end - slot < a.share ? end : slot + a.share;
+    }
+    if (begin >= end) return;
     const index_t home = static_cast<index_t>(bin);
     const index_t hx = home % nx, hy = (home / nx) % ny, hz = home / (nx * ny);
     const int lane = lane_id();
@@ -771,7 +823,7 @@ __global__ void __launch_bounds__(kSearchWaves * kWave) search_pairs_kernel(Sear
     SearchRange range = search_range(a, hx, hy, hz, nx, ny, nz, lane);
     if (!kFull && range.lo <= begin)
     {
-        // a half list alone needs no candidate up to the bin's first atom
+        // a half list alone needs no candidate up to the block's first atom
         const index_t cut =
             range.lo + range.length <= begin + 1 ? range.length : begin + 1 - range.lo;
         range.lo += cut;
@@ -785,7 +837,7 @@ __global__ void __launch_bounds__(kSearchWaves * kWave) search_pairs_kernel(Sear
         tile.to_slot[lane] = range.lo - (inclusive - range.length);
         tile.range_shift[lane] = range.shift;
     }
-    // the box of the bin's atoms, found by the first wave
+    // the box of the block's atoms, found by the first wave
     if (threadIdx.x < kWave)
     {
         T low[3], high[3];
@@ -1121,6 +1173,9 @@ void launch_search(const T* cell, T radius_squared, const ndn_neighbor_buffers& 
     a.dims = b.dims;
     a.cell = cell;
     a.radius_squared = radius_squared;
+    a.atom_bin = b.atom_bin;
+    a.num_atoms = n;
+    a.share = search_share(n);
     a.bin_slots = b.bin_slots;
     a.pair_counts = b.pair_counts;
     a.full_counts = b.full_counts;
@@ -1132,7 +1187,7 @@ void launch_search(const T* cell, T radius_squared, const ndn_neighbor_buffers& 
     a.full_capacity = b.full_capacity;
     a.rebuild = rebuild;
     a.status = b.status;
-    const unsigned blocks = static_cast<unsigned>(bins);
+    const unsigned blocks = static_cast<unsigned>(bins + (b.num_atoms + a.share - 1) / a.share);
     if (full)
         search_pairs_kernel<T, true, kFill><<<blocks, kSearchWaves * kWave, 0, stream>>>(a);
     else

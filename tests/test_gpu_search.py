@@ -98,3 +98,34 @@ def test_scan_of_many_slices(device, n):
     padded[:n] = counts
     np.testing.assert_array_equal(np.diff(slices), 64 * padded.reshape(-1, 64).max(axis=1))
     assert slices[0] == 0 and counts.sum() == 2 * ref.pair_total
+
+
+@pytest.mark.parametrize("dtype,npdt", [(torch.float32, np.float32), (torch.float64, np.float64)])
+@pytest.mark.parametrize("shift", [0, 1, 37])
+def test_bins_of_more_atoms_than_a_block_takes(device, dtype, npdt, shift):
+    """Bins that hold around one, two and three blocks' share of centers (64), and one that holds
+    many tiles of candidates, at slots before and after a multiple of the share."""
+    rng = np.random.default_rng(shift)
+    width, per = 1.0, 6
+    cell = np.full(3, per * width * 1.001).astype(npdt)
+    crowded = {(1, 1, 1): 63, (3, 1, 1): 64, (5, 1, 2): 65, (0, 3, 0): 127, (2, 3, 5): 128,
+               (4, 4, 3): 129, (5, 5, 5): 192, (3, 3, 2): 193, (0, 0, 3): 2500}
+    x = [(np.array(bin) + rng.uniform(0.05, 0.95, (count, 3))) * width
+         for bin, count in crowded.items()]
+    x.append(np.full((shift, 3), 0.5) + rng.uniform(-0.3, 0.3, (shift, 3)))  # in the first bin
+    x.append(rng.uniform(0, per * width, (700, 3)))
+    x = rng.permutation(np.concatenate(x))
+    wrapped, _ = on.wrap(x.astype(npdt), cell)
+    ref = on.build(wrapped, cell, npdt(width), capacity_multiplier=1.25)
+    for full in (True, False):
+        nl = NeighborList(width, full=full)
+        nl.allocate(torch.tensor(x, dtype=dtype, device=device),
+                    torch.tensor(cell, dtype=dtype, device=device))
+        buffers = nl._device.buffers
+        assert buffers["bin_counts"].numel() == per**3 + 1
+        occupied = np.diff(buffers["bin_offsets"].cpu().numpy())
+        assert np.sum(occupied > 64) >= 6 and occupied.max() > 2048
+        np.testing.assert_array_equal(nl.tensors().index.cpu().numpy(), ref.pairs)
+        if full:
+            rows = nl.tensors().full
+            assert int(rows.counts.sum()) == 2 * nl.num_pairs
