@@ -240,7 +240,6 @@ def _frame_indices(frames: Tensor, stored: int):
             or frames.dtype not in (torch.int32, torch.int64)):
         return frames, False
     frames = frames.long()
-    # one pass over a handful of numbers: tensor operations would cost an update 25 us
     values = frames.tolist()
     low = min(values, default=0)
     if low < -stored or max(values, default=0) >= stored:
@@ -256,13 +255,21 @@ def batch_gradient(model: Potential, trained: dict[str, Tensor], prepared: _Prep
     """(gradient by name, loss, terms by name) of the mean loss over ``frames``, in chunks of
     ``size`` frames (``training/_fit.py:33-70``): each frame weighs 1/B, so the chunks' sums
     equal the batch's. Raises ``IndexError`` for a frame outside the prepared set."""
+    frames, checked = _frame_indices(frames, prepared.positions.shape[0])
+    parts = _kernel_parts(model, trained, prepared) if checked else None
+    return _batch_gradient(model, parts, trained, prepared, frames, size, weights, channel_scales)
+
+
+def _batch_gradient(model: Potential, parts, trained: dict[str, Tensor], prepared: _Prepared,
+                    frames: Tensor, size: int, weights: dict[str, float],
+                    channel_scales: dict[str, float]):
+    """``batch_gradient`` of frames known to be in range; through the kernels alone with ``parts``
+    (``_kernel_parts``), else through autograd."""
     channels = tuple(prepared.labels)
     leaves = {name: value.detach().requires_grad_(True) for name, value in trained.items()}
     device = prepared.positions.device
     gradient = {name: torch.zeros_like(value) for name, value in trained.items()}
     total_loss, total_terms = None, None
-    frames, checked = _frame_indices(frames, prepared.positions.shape[0])
-    parts = _kernel_parts(model, trained, prepared) if checked else None
     for chunk in _chunks(frames, size):
         chunk = chunk.to(device)
         if parts is not None:
@@ -393,8 +400,10 @@ def fit(model: Potential, train: Dataset, optimizer: torch.optim.Optimizer, *,
     if echo_every is not None:
         print("update loss " + " ".join(channels), flush=True)
     for update, frames in enumerate(batches(len(train), batch_size, updates, seed)):
-        gradient, value, parts = batch_gradient(model, trained, prepared["training"], frames,
-                                                batch_size, weights, channel_scales)
+        # (a batch's frames are in range as they are drawn)
+        kernels = _kernel_parts(model, trained, prepared["training"])
+        gradient, value, parts = _batch_gradient(model, kernels, trained, prepared["training"],
+                                                 frames, batch_size, weights, channel_scales)
         optimizer_step(optimizer, trained, gradient, held)
         if scheduler is not None:
             scheduler.step()
