@@ -767,7 +767,7 @@ __device__ __forceinline__ void prologue_body(const StepArgs<T>& a, const ndn_po
 }
 
 // A model's coefficient table, by the block: LJ rows (sigma^2, 4 eps, 24 eps, the shift at the
-// cutoff), or the table's padded knots [P, K + 2] and spacing [P].
+// cutoff), or the table's padded knots [P, K + 2], spacing [P] and 1 / spacing [P].
 template <typename T>
 __device__ __forceinline__ void write_coefficients(const ndn_potential& pot, void* coefficients)
 {
@@ -810,7 +810,11 @@ __device__ __forceinline__ void write_coefficients(const ndn_potential& pot, voi
                 out = value(column - 1);
             padded[i] = out;
         }
-        for (int row = threadIdx.x; row < rows; row += blockDim.x) spacing_out[row] = spacing[row];
+        for (int row = threadIdx.x; row < rows; row += blockDim.x)
+        {
+            spacing_out[row] = spacing[row];
+            spacing_out[rows + row] = T(1) / spacing[row];
+        }
     }
 }
 

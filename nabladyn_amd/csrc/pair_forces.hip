@@ -43,7 +43,7 @@ __global__ void lj_rows_kernel(const T* __restrict__ sigma, const T* __restrict_
     out[row] = LJRow<T>{s2, T(4) * e, T(24) * e, T(4) * e * (p6 * p6 - p6)};
 }
 
-// [P, K + 2] padded knots and the spacing (potential/_tabulated/_potential.py:79-82).
+// [P, K + 2] padded knots, the spacing and its reciprocal (potential/_tabulated/_potential.py:79-82).
 template <typename T>
 __global__ void table_pad_kernel(const T* __restrict__ table, const T* __restrict__ spacing,
                                  int rows, int knots, T* __restrict__ padded,
@@ -51,7 +51,11 @@ __global__ void table_pad_kernel(const T* __restrict__ table, const T* __restric
 {
     const std::int64_t index = static_cast<std::int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
     const std::int64_t width = knots + 2;
-    if (index < rows) spacing_out[index] = spacing[index];
+    if (index < rows)
+    {
+        spacing_out[index] = spacing[index];
+        spacing_out[rows + index] = T(1) / spacing[index];
+    }
     if (index >= rows * width) return;
     const std::int64_t row = index / width;
     const std::int64_t column = index % width;
@@ -498,7 +502,7 @@ std::int64_t coefficient_bytes(const ndn_potential* pot, int element)
     if (pot->kind == NDN_LJ)
         bytes = rows * 4 * element;
     else
-        bytes = rows * (pot->knots + 2) * element + rows * element;
+        bytes = rows * (pot->knots + 2) * element + 2 * rows * element;
     return (bytes + 255) / 256 * 256;
 }
 

@@ -129,7 +129,7 @@ struct Table
 {
     const T* __restrict__ padded;        // [P, K + 2]
     const T* __restrict__ start;         // [P]
-    const T* __restrict__ spacing;       // [P]
+    const T* __restrict__ spacing;       // [2, P]: the spacings, then 1 / spacing
     const std::int64_t* __restrict__ types;
     int num_types;
     int knots;                           // K
@@ -143,10 +143,12 @@ struct Table
     {
         // r and the knot coordinate are the reference's: its square root, subtraction and
         // division, each correctly rounded (pair_distance; the quotient is a product with 1/h
-        // corrected by its remainder), so t and the segment are the reference's bits
+        // corrected by its remainder, which is the quotient's rounding when 1/h is correctly
+        // rounded itself, as a hardware reciprocal with Newton steps is not for every h), so t
+        // and the segment are the reference's bits
         const T r = pair_distance(r2);
         const T h = spacing[row_index];
-        const T inverse_h = refined_reciprocal(h);
+        const T inverse_h = spacing[num_types * (num_types + 1) / 2 + row_index];
         const T offset = r - start[row_index];
         const T q = offset * inverse_h;
         const T x = fma(fma(-q, h, offset), inverse_h, q);
