@@ -2204,13 +2204,18 @@ __device__ __forceinline__ index_t xcd_brick(index_t bricks, const Launch launch
 
 // The LDS of a brick's block, one dynamic allocation: the halo (positions and types; entry 0 the
 // far point) from offset 0, so a neighbor's address is its local index times 16 (32 in fp64),
-// then the brick's runs and the block's sums.
+// then the brick's runs and one of the block's sums. The eight sums of a step that needs the
+// virial take the halo's place once the walk is done: room of their own would come off the
+// largest halo that a block may hold.
 struct BrickShared
 {
     index_t run_first[kMaxBrickRuns];
     index_t run_rows[kMaxBrickRuns + 1];
-    double sums[8 * 16];
+    double sums[16];
 };
+
+// Eight sums over up to 16 waves (block_sums).
+constexpr std::size_t kBrickSumBytes = 8 * 16 * sizeof(double);
 
 // Bytes of a block's LDS past the halo.
 constexpr std::size_t kBrickSharedBytes = (sizeof(BrickShared) + 15) / 16 * 16;
@@ -2218,7 +2223,9 @@ constexpr std::size_t kBrickSharedBytes = (sizeof(BrickShared) + 15) / 16 * 16;
 template <typename T>
 __host__ __device__ __forceinline__ std::size_t halo_bytes(std::int64_t halo_capacity)
 {
-    return static_cast<std::size_t>(halo_capacity + 1) * sizeof(typename Vec4<T>::type);
+    const std::size_t bytes =
+        static_cast<std::size_t>(halo_capacity + 1) * sizeof(typename Vec4<T>::type);
+    return bytes > kBrickSumBytes ? bytes : kBrickSumBytes;
 }
 
 // Dynamic LDS of a brick's block: the halo (with the sentinel) and the block's bookkeeping (a
@@ -2582,14 +2589,15 @@ __device__ __forceinline__ void force_body(const StepArgs<T>& a, const Launch la
             }
         }
     }
-    // all of the block's sums behind one barrier: with one sum after another the seven of a step
-    // that needs the virial took 2 us of its 40 (10,007 atoms, fp64, NPT)
+    // all of the block's sums behind one barrier (one sum after another, the seven of a step that
+    // needs the virial took 2 us of its 40 at 10,007 atoms, fp64, NPT)
     const int k = threadIdx.x;
     if (kVirial)
     {
         double terms[8] = {kEnergy ? energy_sum : 0.0, w_sum[0], w_sum[1], w_sum[2], w_sum[3],
                            w_sum[4], w_sum[5], kinetic};
-        const double sum = block_sums(terms, sh->sums);
+        __syncthreads();  // no thread reads the halo any more
+        const double sum = block_sums(terms, reinterpret_cast<double*>(dynamic_shared));
         if (k < 8) out[k * column] = sum;
     }
     else

@@ -8,6 +8,7 @@ import pytest
 import torch
 
 from nabladyn_amd import md, potential
+from nabladyn_amd.md._simulation import halo_limit
 
 pytestmark = pytest.mark.gpu
 
@@ -57,3 +58,16 @@ def test_a_row_overflow_moves_the_whole_frame(device, dtype, n):
     np.testing.assert_array_equal(sim.slot_masses.cpu().numpy(), masses.cpu().numpy()[ids])
     got = sim.positions.cpu().numpy()
     np.testing.assert_allclose(got, (x + v * 0.4)[ids], rtol=0, atol=2e-4)
+
+
+@pytest.mark.parametrize("dtype,point", [(torch.float32, 16), (torch.float64, 32)])
+def test_a_halo_may_take_half_a_units_lds(device, dtype, point):
+    """The largest halo: half of a compute unit's 160 KB, less 656 bytes of a block's own. 6,000 atoms
+    of some 200 bricks take all of it, and run."""
+    limit = halo_limit(dtype)
+    assert limit >= (160 * 1024 // 2 - 656) // point - 1
+    sim, x, v, _ = _gathering(device, dtype, 6000, 0.4 * 19, 0.95, 20)
+    assert sim._neighbors.halo_capacity == min(limit, 6000)
+    sim.run(20)
+    got = sim.state().positions.cpu().numpy()
+    np.testing.assert_allclose(got, x + v * 0.08, rtol=0, atol=2e-4)
