@@ -2937,7 +2937,10 @@ void allow_shared(Kernel kernel, std::size_t bytes)
 // 2,000 26.1 / 22.6 / 24.0, 4,096 27.3 / 24.0 / 29.2, 32,768 34.7 / 32.5 / -, 100,000 (skin 0.2)
 // 51.0 / 49.5 / - and (skin 0.1) 47.1 / 47.8 / -: past some 65,536 atoms the one block's sort
 // costs a build what the launches cost the steps between. (One block that also filled took 36 us
-// at 512 atoms and 55 at 2,000.)
+// at 512 atoms and 55 at 2,000.) Both only while the sub-bins' counts fit a block's LDS, of whose
+// 160 KB the kernel's own variables take some hundred bytes: 36,863 sub-bins. A dilute box of more
+// takes the separate launches (512 atoms in 125,000 sub-bins: 32 us a step, 144 with one block for
+// the whole build).
 constexpr std::int64_t kWholeSort = 1024;
 constexpr std::int64_t kOneBlockSort = 65536;
 constexpr std::size_t kSortBytes = 144 * 1024;
