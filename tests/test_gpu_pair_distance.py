@@ -1,9 +1,10 @@
-"""The fp64 root, quotient and reciprocals of the pair kernels: isolated pairs over the whole range
-of distances, each pair's force against numpy's correctly rounded root and division.
+"""The fp64 root and reciprocals of the pair kernels: isolated pairs over the whole range of
+distances, each pair's force against numpy's correctly rounded root and division.
 
 The table is linear between knots of a power-of-two spacing, so a pair's force is its slope times
 the unit vector, in a handful of roundings: 8 of 2^-53 relative. An atom pair is along x, so the
-force's x is the slope itself to within those."""
+force's x is the slope itself to within those. (A linear table's slope is the same wherever the
+knot coordinate falls: test_gpu_knot_coordinate.py has the quotient that gives it.)"""
 
 import numpy as np
 import pytest
