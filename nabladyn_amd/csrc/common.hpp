@@ -174,8 +174,10 @@ __device__ __forceinline__ V block_sum(V value, V* shared)
 
 // The block's sums of N values behind one barrier: thread k < N returns the k-th, in the order of
 // block_sum (any other thread a meaningless value). `shared` holds 16 N values, which no other use
-// of it may touch before a barrier.
-template <int N, typename V>
+// of it may touch before a barrier. With kTakes the values take the place of data that other
+// waves may still read: a barrier comes before they are written, after the waves' own sums, so
+// that a wave which is done early forms them while the others go on.
+template <bool kTakes, int N, typename V>
 __device__ __forceinline__ V block_sums(V (&values)[N], V* shared)
 {
     const int lane = lane_id();
@@ -185,8 +187,14 @@ __device__ __forceinline__ V block_sums(V (&values)[N], V* shared)
     for (int k = 0; k < N; ++k)
     {
         values[k] = wave_sum(values[k]);
-        if (lane == 0) shared[16 * k + wave] = values[k];
+        // held here: the compiler would move the shuffles past the barrier, where every wave of
+        // the block waits for them (a step of 150,000 atoms at constant pressure 95 -> 103 us)
+        if (kTakes) asm volatile("" : "+v"(values[k]));
     }
+    if (kTakes) __syncthreads();
+    if (lane == 0)
+#pragma unroll
+        for (int k = 0; k < N; ++k) shared[16 * k + wave] = values[k];
     __syncthreads();
     V sum = 0;
     if (threadIdx.x < N)

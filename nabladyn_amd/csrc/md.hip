@@ -2596,15 +2596,14 @@ __device__ __forceinline__ void force_body(const StepArgs<T>& a, const Launch la
     {
         double terms[8] = {kEnergy ? energy_sum : 0.0, w_sum[0], w_sum[1], w_sum[2], w_sum[3],
                            w_sum[4], w_sum[5], kinetic};
-        __syncthreads();  // no thread reads the halo any more
-        const double sum = block_sums(terms, reinterpret_cast<double*>(dynamic_shared));
+        const double sum = block_sums<true>(terms, reinterpret_cast<double*>(dynamic_shared));
         if (k < 8) out[k * column] = sum;
     }
     else
     {
         // E or K alone, which thread 0 holds
         double terms[1] = {kKick ? kinetic : energy_sum};
-        const double sum = block_sums(terms, sh->sums);
+        const double sum = block_sums<false>(terms, sh->sums);
         if (k < 8) out[(kKick ? (k + 7) % 8 : k) * column] = k == 0 ? sum : 0.0;
     }
 }
