@@ -284,8 +284,9 @@ int ndn_frames_loss(int dtype, int64_t frames, int64_t num_atoms, int64_t stored
  * (code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc). No
  * counterpart in the reference. Its scratch (the potential's coefficients, then 64 bytes per
  * block of the pair launch, at most 2,048 blocks) is a static device array of
- * NDN_PAIR_EFW_NOALLOC_SCRATCH_BYTES per GPU, held until the process ends; a call whose
- * potential and list need more is refused with NDN_ERR_ARGUMENT. It calls no allocator.
+ * NDN_PAIR_EFW_NOALLOC_SCRATCH_BYTES and a quarter more per GPU, held until the process ends; a
+ * call whose potential (a table's rows of K + 3 numbers) and list need more than the former is
+ * refused with NDN_ERR_ARGUMENT. It calls no allocator.
  * Nothing in the scratch needs clearing between calls (each call writes what it reads), but
  * every call on one GPU shares that GPU's array: calls that overlap on one GPU (two streams,
  * two threads) race and must be serialised by the caller. */

@@ -495,14 +495,14 @@ int check_potential(const ndn_potential* pot, std::int64_t num_atoms)
     return NDN_OK;
 }
 
-std::int64_t coefficient_bytes(const ndn_potential* pot, int element)
+std::int64_t coefficient_bytes(const ndn_potential* pot, int element, bool reciprocals)
 {
     const std::int64_t rows = static_cast<std::int64_t>(pot->num_types) * (pot->num_types + 1) / 2;
     std::int64_t bytes;
     if (pot->kind == NDN_LJ)
         bytes = rows * 4 * element;
     else
-        bytes = rows * (pot->knots + 2) * element + 2 * rows * element;
+        bytes = rows * (pot->knots + 2) * element + (reciprocals ? 2 : 1) * rows * element;
     return (bytes + 255) / 256 * 256;
 }
 
@@ -815,7 +815,11 @@ int pair_efw_frames_impl(const void* positions, const void* cells, std::int64_t 
 // library runs on holds its own copy until the process ends. Host code never passes this name
 // to a kernel (on the host it is a stand-in, not a device address); it passes the address
 // hipGetSymbolAddress returns for the device, looked up once per device and kept.
-static __device__ __align__(256) unsigned char scratch[NDN_PAIR_EFW_NOALLOC_SCRATCH_BYTES];
+//
+// A quarter more than the stated bytes: the reciprocals of a table's spacings, which the limit does
+// not count, are at most a seventh of them (four knots a row at least).
+static __device__ __align__(256) unsigned char
+    scratch[NDN_PAIR_EFW_NOALLOC_SCRATCH_BYTES + NDN_PAIR_EFW_NOALLOC_SCRATCH_BYTES / 4];
 
 constexpr int kMaxDevices = 64;
 std::mutex scratch_mutex;
@@ -1005,7 +1009,7 @@ extern "C" int ndn_pair_efw_noalloc(int dtype, const void* positions, const void
     NDN_REQUIRE(num_atoms >= 1 && num_atoms <= INT32_MAX, "N must satisfy 1 <= N < 2**31");
     NDN_REQUIRE(capacity >= 1 && capacity <= INT32_MAX, "pairs must be [2, C] with int32 C");
     const int element = dtype == NDN_F32 ? 4 : 8;
-    const std::int64_t needed = coefficient_bytes(pot, element) +
+    const std::int64_t needed = coefficient_bytes(pot, element, false) +
                                 static_cast<std::int64_t>(half_blocks(capacity)) * 8 *
                                     static_cast<std::int64_t>(sizeof(double));
     if (needed > NDN_PAIR_EFW_NOALLOC_SCRATCH_BYTES)

@@ -138,7 +138,8 @@ __device__ __forceinline__ void store_partials(double energy, const T* w, double
     }
 }
 
-std::int64_t coefficient_bytes(const ndn_potential* pot, int element);
+// Bytes of a potential's coefficients; without the reciprocals of a table's spacings on request.
+std::int64_t coefficient_bytes(const ndn_potential* pot, int element, bool reciprocals = true);
 int check_potential(const ndn_potential* pot, std::int64_t num_atoms);
 
 template <typename T>

@@ -72,3 +72,30 @@ def test_noalloc_equals_workspace_entry_point(device, dtype, kind, tol):
         assert torch.equal(got[2], want[2])
         scale = float(want[1].abs().max())
         assert float((got[1] - want[1]).abs().max()) <= tol * scale
+
+
+@pytest.mark.parametrize("dtype,element,tol", [(torch.float32, 4, 1e-6), (torch.float64, 8, 1e-13)])
+def test_the_largest_table_the_scratch_takes(device, dtype, element, tol):
+    """Rows of K + 3 numbers, rounded up to 256 bytes, and a 64-byte slot a block fill the scratch:
+    the largest table is taken, one more knot is refused."""
+    n = 64
+    x, cell, pairs, _ = _system(n, 2.9, 3, dtype, device, "lj")
+    slots = 64 * min(2048, -(-pairs.index.shape[1] // 256))
+    room = ((1 << 20) - slots) // 256 * 256
+    for knots, taken in ((room // element - 3, True), (room // element - 2, False)):
+        r = np.linspace(0.3, 1.0, knots)
+        table = (1.0 - r) ** 2 / 0.49
+        table[-1] = 0.0
+        model = potential.tabulated(
+            atom_types=torch.zeros(n, dtype=torch.int64, device=device),
+            table=torch.tensor(table[None], dtype=dtype, device=device),
+            start=torch.tensor([0.3], dtype=dtype, device=device), cutoff=1.0)
+        if not taken:
+            with pytest.raises(_native.NativeError, match="more than its"):
+                _noalloc(x, cell, pairs, model)
+            continue
+        got = _noalloc(x, cell, pairs, model)
+        want = quantity._evaluate(model, x, cell, pairs._replace(full=None), energy=True,
+                                  forces=True, virial=True)
+        assert torch.equal(got[0], want[0]) and torch.equal(got[2], want[2])
+        assert float((got[1] - want[1]).abs().max()) <= tol * float(want[1].abs().max())
